@@ -74,14 +74,15 @@ struct bread_decode_sync {
 
 // Workspace of the grouped (multi-token) path, sized for max_tokens.
 struct bread_grouped_ws {
-    void *xhi = nullptr, *xlo = nullptr;  // activations as hi/lo fp16 [max_tokens][H]
+    int cus = 0;                          // compute units of the device
+    void *xop = nullptr;                  // activations as hi/lo fp16 in operand order [max_tokens][H/256][2][256]
+    void *xsum = nullptr;                 // their sub-block sums, hi/lo fp16 [max_tokens][H/256][2][8]
     int *xexp = nullptr;                  // row scale exponents [max_tokens]
     int *pair_tok = nullptr;              // token of each expert-sorted pair [max_tokens*(K+1)]
     int *pos_of = nullptr;                // sorted position of pair (t, k) [max_tokens*K]
-    void *tiles = nullptr;                // M-tiles of the expert GEMMs
-    int *n_tiles = nullptr;
-    int *work = nullptr;                  // per-XCD work lists of the two expert GEMMs
-    int *n_work = nullptr;                // their lengths [2][8]
+    void *tiles = nullptr;                // tiles of the expert GEMMs
+    int *n_tiles = nullptr;               // routed tiles, and all with the shared expert's
+    float *h = nullptr;                   // SwiGLU rows by tile [tiles][32][Imax]
     float *eo = nullptr;                  // expert outputs by pair [max_tokens*(K+1)][H]
 };
 

@@ -1,33 +1,23 @@
 // moe_grouped.hip — the multi-token MoE path (batched decode, speculative
 // verify, prefill chunks): tokens bucketed by expert, the expert products as
-// grouped GEMMs on the gfx950 matrix cores with the K-quant weights
-// dequantised in registers, and a combine in the reference order.
+// grouped GEMMs on the gfx950 matrix cores with the K-quant weights unpacked
+// in registers, and a combine in the reference order.
 //
 // The reference has no multi-token MoE: prefill runs token by token
 // (main.cu:615-639) and speculative verify is sequential
 // (main_speculative.cu:477-497).  Per token the result is the MoE block of
 // one_layer_forward (one_layer.cu:1800-1986; CPU form 1413-1471).
 //
-// Numerics.  MFMA operands are fp16 with fp32 accumulation.  A bf16 operand
-// (8-bit significand) leaves about 4e-3 relative L2 error on one expert's
-// output, above the 1e-3 bound of this path; fp16 weights (one rounding of
-// the exact K-quant value) times activations carried as two fp16 terms
-// (hi + lo, 22 significant bits) leave about 4e-4.  Before the split each
-// activation row is scaled by a power of two so that its largest magnitude
-// lies in [2^13, 2^14) (exact, undone on the fp32 result): SwiGLU outputs
-// reach 1e5 at the synthetic weight scale, beyond fp16's range.
-//
-// Weight dequantisation, one instruction per weight: a byte holding a 4- or
-// 6-bit code q becomes the fp16 value 1024 + q by byte permutation (0x64 in
-// the high byte), and v_fma_mix{lo,hi}_f16 computes (1024 + q) * d + c in
-// fp32 with c = -(1024 * d + m) and rounds once to fp16, giving d * q - m
-// (Q4_K, dequant_q4k_cpu.c:117-118) or d * sc * (q - 32) (Q6_K, c = -1056 *
-// d * sc, dequant_q4k_cpu.c:160-165).
-//
-// Expert GEMMs use v_mfma_f32_32x32x16_f16 with the weights as the M side
-// (32 rows) and the M-tile's 32 (token, expert) pairs as the N side: each
-// dequantised weight fragment meets 32 tokens in one instruction, and each
-// activation fragment read from LDS serves 32 weight rows.
+// Numerics.  MFMA operands are fp16 with fp32 accumulation, and every
+// product is exact.  A weight enters as its integer part: sc * q (Q4_K,
+// <= 63 * 15) or sc * (q - 32) (Q6_K, |.| <= 4096: exact up to 2048 and for
+// even values; the odd ones above are rounded to even in layers of the
+// reference GPU path's types and carried by a second operand in the others,
+// which ran in fp32 before).  Activations are two fp16 terms (hi + lo, 22
+// significant bits) after a power-of-two row scale into [2^13, 2^14) (exact,
+// undone on the fp32 result).  The superblock scale d, and for Q4_K the min
+// term dmin * sum_j m_j * (sum of x over sub-block j), are applied to the
+// fp32 sums.
 //
 // Kernels per layer, stream-ordered:
 //   k_route_seq   router logits in the reference's sequential order
@@ -35,18 +25,20 @@
 //   k_mt_topk_xprep  one workgroup per token: softmax / top-k /
 //                 renormalisation with the host's arithmetic (routing
 //                 bit-identical to the reference's), and the activation
-//                 preparation: row scale, hi/lo fp16 activations in the
-//                 gate/up operand order, shared-gate logit
+//                 preparation: row scale, hi/lo fp16 activations in MFMA
+//                 operand order, sub-block sums, shared-gate logit
 //   k_mt_bucket   one workgroup: expert histogram, token lists by expert,
-//                 M-tiles of 32 pairs
-//   k_mt_gateup   per (M-tile, 128 rows): gate and up GEMMs, SwiGLU
-//   k_mt_down     per (M-tile, 512 rows): the tile's SwiGLU rows split into
-//                 hi/lo fp16 with a row scale, then the down GEMM
+//                 tiles of 32 pairs
+//   k_gateup      per (tile, 128 rows): gate and up GEMMs and SwiGLU
+//   k_down_gg     per (tile, 512 rows): the tile's SwiGLU rows split into hi/lo
+//                 fp16 with a row scale, then the down GEMM
 //   k_mt_combine  per token: shared expert, then routed experts in rank order
 // The shared expert is expert index E with every token, so both GEMMs treat
 // it like a routed expert with its own weights.
 #include <float.h>
 #include <stdlib.h>
+
+#include <type_traits>
 
 #include "bread_internal.h"
 #include "bread_device.h"
@@ -55,19 +47,17 @@
 
 namespace {
 
-constexpr int MT = 32;                           // (token, expert) pairs per M-tile
-constexpr int GU_WAVES = 8;                      // one 32-row gate or up block per wave
-constexpr int GU_ROWS = GU_WAVES / 2 * 32;       // SwiGLU rows per gate/up workgroup
-constexpr int DN_WAVES = 8, DN_BLOCKS = 2;       // 32-row down blocks per wave
-constexpr int DN_ROWS = DN_WAVES * DN_BLOCKS * 32;  // output rows per down workgroup
-constexpr int MAX_INTER = 512;                   // largest intermediate size the LDS plan holds
-constexpr int NXCD = 8;                          // L2 domains; workgroup L runs on XCD L % 8
-constexpr int SEG = 4;                           // tiles of one expert kept on one XCD
-constexpr uint32_t MAGIC = 0x64646464u;          // fp16 0x64xx = 1024 + xx
+constexpr int MT = 32;           // (token, expert) pairs per tile
+constexpr int MAX_INTER = 512;   // largest intermediate size of this path
+constexpr int NXCD = 8;          // L2 domains; workgroup L runs on XCD L % 8
+constexpr int GG_WAVES = 4;
+constexpr int GG_THREADS = GG_WAVES * WAVE;
+constexpr int GU_ROWS = 32 * GG_WAVES;       // gate and up rows of a gate/up workgroup
+constexpr int DN_WAVES = 8, DN_BLOCKS = 2;   // 32-row blocks of a wave of the down kernel
+constexpr int DN_ROWS = 32 * DN_WAVES * DN_BLOCKS;
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 struct MtTile {
@@ -77,39 +67,9 @@ struct MtTile {
     int pad;
 };
 
-struct MtArgs {
-    bread_moe_layer_t L;
-    uint32_t *err;           // device error word of the context
-    int H, I, Ish, Imax, E, K, T;
-    const uint4 *xhi, *xlo;  // [T][H/8] units of 8 fp16, gate/up operand order
-    const int *xexp;         // [T] row scale exponents
-    const int *pair_tok;     // [T*K + T] token of each sorted pair
-    const MtTile *tiles;
-    const int *n_tiles;
-    const int *work_gu, *work_dn;  // per-XCD work items (tile << 8 | chunk) of the two GEMMs
-    const int *n_work;             // [2][NXCD] items per XCD (gate/up, down)
-    int slots_gu, slots_dn;        // list capacity per XCD
-    float *h;                // [T*K + T][Imax] SwiGLU outputs by pair
-    float *eo;               // [T*K + T][H] expert outputs by pair
-};
-
-__device__ __forceinline__ void lds_load16(const void *src, void *lds_wave_base)
-{
-    __builtin_amdgcn_global_load_lds(src, lds_wave_base, 16, 0, 0);
-}
-
 __device__ __forceinline__ uint32_t comp(const uint4 &q, int i)
 {
     return i == 0 ? q.x : (i == 1 ? q.y : (i == 2 ? q.z : q.w));
-}
-
-// s_waitcnt with vmcnt <= n (n < 16) and the other counters unconstrained
-// (gfx9 encoding: vmcnt[3:0], expcnt[6:4], lgkmcnt[11:8]).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt()
-{
-    static_assert(N >= 0 && N < 16, "vmcnt");
-    __builtin_amdgcn_s_waitcnt(N | (7 << 4) | (15 << 8));
 }
 
 // Exponent e with max_abs * 2^-e in [2^13, 2^14); 0 for an all-zero or
@@ -133,142 +93,60 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t 
     lo = (uint32_t)__builtin_bit_cast(uint16_t, la) | ((uint32_t)__builtin_bit_cast(uint16_t, lb) << 16);
 }
 
-__device__ __forceinline__ void split8(const float (&v)[8], int e, uint4 &hi, uint4 &lo)
+// ---------------------------------------------------------------------------
+// Operand order.  v_mfma_f32_32x32x16_f16 with 32 tokens as the M side and 32
+// weight rows as the N side: lane (r = lane % 32, g = lane / 32) holds weight
+// row r and token r, eight K elements of the step.  K is relabelled so that
+// one order serves Q4_K and Q6_K and a lane's bytes are contiguous: lane half
+// g takes the elements 128 g .. 128 g + 127 of a superblock, and step s = 8 pp
+// + k of 16 takes of those
+//   b + {0, 2, 1, 3} and b + 32 + {0, 2, 1, 3},  b = 128 g + 64 pp + 4 k.
+// Q4_K: the two quads are the low and high nibbles of one qs dword
+// (dequant_q4k_cpu.c:111-121); Q6_K: a nibble each of one dword of the two ql
+// ranges with two bits each of one qh dword (dequant_q4k_cpu.c:155-170).
+// {0, 2, 1, 3}: a mask with 16-bit period picks bytes 0 and 2 of a dword, the
+// same mask 8 bits on bytes 1 and 3.  Unit u = 2 s + g of a superblock holds a
+// lane's eight elements of step s.
+// ---------------------------------------------------------------------------
+
+__device__ __forceinline__ int unit_base(int u)
 {
-    split2(ldexpf(v[0], -e), ldexpf(v[1], -e), hi.x, lo.x);
-    split2(ldexpf(v[2], -e), ldexpf(v[3], -e), hi.y, lo.y);
-    split2(ldexpf(v[4], -e), ldexpf(v[5], -e), hi.z, lo.z);
-    split2(ldexpf(v[6], -e), ldexpf(v[7], -e), hi.w, lo.w);
+    return 128 * (u & 1) + 64 * (u >> 4) + 4 * ((u >> 1) & 7);
 }
 
-// Two fp16 values (1024 + q0, 1024 + q1) -> fp16(fp32 (1024 + q) * d + c).
-__device__ __forceinline__ uint32_t mix2(uint32_t q2, float d, float c)
+// Eight elements in operand order (a: b .. b + 3, c: b + 32 .. b + 35),
+// scaled by 2^-e and split.
+__device__ __forceinline__ void split_unit(const float4 &a, const float4 &c, int e, uint4 &hi, uint4 &lo)
 {
-    const half2v h = __builtin_bit_cast(half2v, q2);
-    half2v r;
-    r[0] = (_Float16)__builtin_fmaf((float)h[0], d, c);
-    r[1] = (_Float16)__builtin_fmaf((float)h[1], d, c);
-    return __builtin_bit_cast(uint32_t, r);
+    split2(ldexpf(a.x, -e), ldexpf(a.z, -e), hi.x, lo.x);
+    split2(ldexpf(a.y, -e), ldexpf(a.w, -e), hi.y, lo.y);
+    split2(ldexpf(c.x, -e), ldexpf(c.z, -e), hi.z, lo.z);
+    split2(ldexpf(c.y, -e), ldexpf(c.w, -e), hi.w, lo.w);
 }
 
-// Bytes b0..b3 of v (codes < 256) -> four fp16 weights in byte order,
-// (b0, b1) in r0 and (b2, b3) in r1.
-__device__ __forceinline__ void bytes_to_w(uint32_t v, float d, float c, uint32_t &r0, uint32_t &r1)
+// The same for eight elements already in operand order.
+__device__ __forceinline__ void split_unit_op(const float4 &a, const float4 &c, int e, uint4 &hi, uint4 &lo)
 {
-    r0 = mix2(__builtin_amdgcn_perm(MAGIC, v, 0x07010700u), d, c);
-    r1 = mix2(__builtin_amdgcn_perm(MAGIC, v, 0x07030702u), d, c);
-}
-
-// D[32 weight rows][32 pairs] += W[32][16] * X[16][32].  Lane l holds W row
-// l%32 and X column l%32, K elements 8*(l/32) .. +7 of the step; D register
-// i holds row 8*(i/4) + 4*(l/32) + i%4 of column l%32.
-__device__ __forceinline__ f32x16 mfma32(const uint4 &w, const uint4 &x, f32x16 acc)
-{
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, w), __builtin_bit_cast(half8, x), acc,
-                                                  0, 0, 0);
+    split2(ldexpf(a.x, -e), ldexpf(a.y, -e), hi.x, lo.x);
+    split2(ldexpf(a.z, -e), ldexpf(a.w, -e), hi.y, lo.y);
+    split2(ldexpf(c.x, -e), ldexpf(c.y, -e), hi.z, lo.z);
+    split2(ldexpf(c.z, -e), ldexpf(c.w, -e), hi.w, lo.w);
 }
 
 // ---------------------------------------------------------------------------
-// Gate/up operand order (Q4_K).  Lane (row r = lane%32, group g = lane/32) of
-// a 32-row block reads qs bytes [64g, 64g+64) of each superblock row, i.e.
-// sub-block pairs p = 2g and 2g+1.  K-step s (0..15) of a superblock uses qs
-// dword s%8 of pair p = 2g + s/8: B element j of the lane is superblock
-// element 64p + 4(s%8) + j (j < 4, low nibbles, sub-block 2p) or
-// 64p + 32 + 4(s%8) + (j - 4) (j >= 4, high nibbles, sub-block 2p + 1).
-// The activations are stored in the same order: unit u = 32*sb + 2*s + g of
-// a token row holds those 8 elements.
+// Activation preparation: row scale, the row's units (hi then lo per
+// superblock, [T][H / 256][2][32]) and the sums over the 32-element
+// sub-blocks times 2^-5 (hi and lo unit of eight, [T][H / 256][2]) that the
+// Q4_K min term multiplies; the shared-gate logit.
 // ---------------------------------------------------------------------------
 
-// Packed-fp16 form of the same weights, two per instruction:
-//   t = fma(1024 + q, sc, -1024 sc) = sc * q   (exact: |sc q| <= 945)
-//   w = fma(t, d, fp16(-dmin * m))             (one rounding, as above, plus
-//                                               the fp16 rounding of dmin * m)
-// Valid while d * 945 and dmin * 63 stay inside fp16's range (|d| < 64,
-// |dmin| < 1024), which fp16 weights need anyway; superblocks outside it
-// raise BREAD_DEV_ERR_RANGE.
-struct Q4Pk {
-    half2v sc[4], nsc[4], m[4], d;
-};
-
-__device__ __forceinline__ Q4Pk q4k_lane_pk(const uint4 &hd, uint32_t g)
+__device__ __forceinline__ float xor_add(float v, int m)
 {
-    Q4Pk s;
-    const float dmin = h2f(hd.x >> 16);
-    const _Float16 d16 = __builtin_bit_cast(_Float16, (uint16_t)(hd.x & 0xFFFFu));
-    s.d = half2v{d16, d16};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        uint32_t sc, m;
-        scale_min_k4(4 * g + q, hd.y, hd.z, hd.w, sc, m);
-        const _Float16 scf = (_Float16)(float)sc, nscf = (_Float16)(-1024.f * (float)sc);
-        const _Float16 mf = (_Float16)(-(dmin * (float)m));
-        s.sc[q] = half2v{scf, scf};
-        s.nsc[q] = half2v{nscf, nscf};
-        s.m[q] = half2v{mf, mf};
-    }
-    return s;
+    return v + __shfl_xor(v, m);
 }
-
-__device__ __forceinline__ uint32_t pk_w(uint32_t qb, const Q4Pk &s, int q)
-{
-    const half2v t = __builtin_elementwise_fma(__builtin_bit_cast(half2v, qb), s.sc[q], s.nsc[q]);
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(t, s.d, s.m[q]));
-}
-
-__device__ __forceinline__ bool q4k_pk_ok(const uint4 &hd)
-{
-    const float d = fabsf(h2f(hd.x)), dmin = fabsf(h2f(hd.x >> 16));
-    return d < 64.f && dmin < 1024.f;  // false for NaN
-}
-
-// ---------------------------------------------------------------------------
-// Down operand order (Q6_K).  Lane (row r, group g) of a 32-row block takes
-// half g (elements 128g .. 128g+127) of each superblock row; K-step t (0..15)
-// of the half covers its elements 8t .. 8t+7 (natural order): low nibbles
-// of ql bytes 8t.. (t < 8) or high nibbles of ql bytes 8(t-8).. (t >= 8),
-// with qh bits 2*(t/4) of qh bytes 8(t%4).. and scale sc[8g + t/2]
-// (dequant_q4k_cpu.c:155-170).  Activation unit ((16b + t)*2 + g) of a row
-// holds elements 256b + 128g + 8t .. +7.
-//
-// The lane's bytes are 2-byte aligned (superblocks are 210 bytes), so each
-// range is loaded as whole dwords from the aligned-down address and shifted
-// with v_alignbyte.  Every dword loaded holds a byte of the superblock or of
-// the next one in the same expert block (an expert block ends 16-byte
-// aligned, so a superblock starting at a multiple of 4 is never its last).
-// ---------------------------------------------------------------------------
-
-struct Q6Raw {
-    uint4 ql[4];
-    uint32_t ql4;
-    uint4 qh[2];
-    uint32_t qh2;
-    uint4 sc;
-    uint32_t sc1;
-};
-
-__device__ __forceinline__ void q6k_load(const uint8_t *sb, int g, Q6Raw &R)
-{
-    // aligned down by pointer arithmetic: a pointer rebuilt from an integer
-    // is generic to the compiler, which would emit flat loads (counted on
-    // lgkmcnt too, so every LDS wait would also wait for these)
-    const uint8_t *p = sb - (reinterpret_cast<uintptr_t>(sb) & 3u);
-    const uint8_t *ql = p + 64 * g, *qh = p + 128 + 32 * g, *sc = p + 192;
-#pragma unroll
-    for (int i = 0; i < 4; i++) R.ql[i] = *reinterpret_cast<const uint4 *>(ql + 16 * i);
-    R.ql4 = *reinterpret_cast<const uint32_t *>(ql + 64);
-    R.qh[0] = *reinterpret_cast<const uint4 *>(qh);
-    R.qh[1] = *reinterpret_cast<const uint4 *>(qh + 16);
-    R.qh2 = *reinterpret_cast<const uint32_t *>(qh + 32);
-    R.sc = *reinterpret_cast<const uint4 *>(sc);
-    R.sc1 = *reinterpret_cast<const uint32_t *>(sc + 16);
-}
-
-// ---------------------------------------------------------------------------
-// Activation preparation and router
-// ---------------------------------------------------------------------------
 
 __device__ __forceinline__ void mt_xprep(int t, const float *__restrict__ x, const uint16_t *__restrict__ shg, int H,
-                                         uint4 *__restrict__ xhi, uint4 *__restrict__ xlo, int *__restrict__ xexp,
+                                         uint4 *__restrict__ xop, uint4 *__restrict__ xsum, int *__restrict__ xexp,
                                          float *__restrict__ gsh)
 {
     __shared__ float smax[4], sdot[4];
@@ -297,29 +175,42 @@ __device__ __forceinline__ void mt_xprep(int t, const float *__restrict__ x, con
         xexp[t] = e;
         if (gsh) gsh[t] = shg ? (sdot[0] + sdot[1]) + (sdot[2] + sdot[3]) : 0.f;
     }
+    // one unit a thread and pass; H / 8 is a multiple of 32, so the 32 lanes
+    // of a superblock are active together
     const int nu = H / 8;
     for (int u = threadIdx.x; u < nu; u += 256) {
-        const int sb = u >> 5, s = (u >> 1) & 15, g = u & 1;
-        const int b = QK * sb + 64 * (2 * g + (s >> 3)) + 4 * (s & 7);
-        const float4 lo4 = *reinterpret_cast<const float4 *>(xt + b);
-        const float4 hi4 = *reinterpret_cast<const float4 *>(xt + b + 32);
-        const float v[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+        const int sb = u >> 5, b = QK * sb + unit_base(u & 31);
+        const float4 a = *reinterpret_cast<const float4 *>(xt + b);
+        const float4 c = *reinterpret_cast<const float4 *>(xt + b + 32);
         uint4 h, l;
-        split8(v, e, h, l);
-        xhi[(size_t)t * nu + u] = h;
-        xlo[(size_t)t * nu + u] = l;
+        split_unit(a, c, e, h, l);
+        uint4 *o = xop + ((size_t)t * (H / QK) + sb) * 64;
+        o[u & 31] = h;
+        o[32 + (u & 31)] = l;
+        // sub-blocks j = 4 g + 2 pp (a) and j + 1 (c): sums over k
+        float sa = ldexpf((a.x + a.y) + (a.z + a.w), -e - 5), sc = ldexpf((c.x + c.y) + (c.z + c.w), -e - 5);
+        sa = xor_add(xor_add(xor_add(sa, 2), 4), 8);
+        sc = xor_add(xor_add(xor_add(sc, 2), 4), 8);
+        if ((u & 0xE) == 0) {
+            uint32_t hh, ll;
+            split2(sa, sc, hh, ll);
+            uint32_t *so = reinterpret_cast<uint32_t *>(xsum + ((size_t)t * (H / QK) + sb) * 2);
+            const int j2 = 2 * (u & 1) + ((u >> 4) & 1);  // j / 2
+            so[j2] = hh;
+            so[4 + j2] = ll;
+        }
     }
 }
 
-// Per token, one workgroup: the activation preparation (row scale, hi/lo
-// fp16 activations in the gate/up operand order, shared-gate logit) and, on
+// Per token, one workgroup: the activation preparation (row scale, operand
+// units, shared-gate logit) and, on
 // wave 0, softmax / top-k / renormalisation with the host's arithmetic on
 // the router logits (route_dev.h topk_wave_exact).
 template <int MAXV>
 __global__ __launch_bounds__(256) void k_mt_topk_xprep(const float *__restrict__ logits, int E, int K,
                                                        int32_t *__restrict__ idx, float *__restrict__ w,
                                                        const float *__restrict__ x, const uint16_t *__restrict__ shg,
-                                                       int H, uint4 *__restrict__ xhi, uint4 *__restrict__ xlo,
+                                                       int H, uint4 *__restrict__ xop, uint4 *__restrict__ xsum,
                                                        int *__restrict__ xexp, float *__restrict__ gsh)
 {
     __shared__ __attribute__((aligned(16))) float s_e[WAVE * MAXV];
@@ -333,7 +224,7 @@ __global__ __launch_bounds__(256) void k_mt_topk_xprep(const float *__restrict__
             w[(size_t)t * K + lane_id()] = wk;
         }
     }
-    mt_xprep(t, x, shg, H, xhi, xlo, xexp, gsh);
+    mt_xprep(t, x, shg, H, xop, xsum, xexp, gsh);
 }
 
 // ---------------------------------------------------------------------------
@@ -367,17 +258,15 @@ __device__ __forceinline__ void block_scan2(int a, int b, int *wsa, int *wsb, in
 
 // Pairs (token t, rank k) sorted by expert; the shared expert's pairs
 // (every token in order) follow at T*K.  pos_of[t*K + k] = sorted position
-// (-1 for an index outside [0, E), which the combine skips).
+// (-1 for an index outside [0, E), which the combine skips).  Tiles: the
+// routed experts' in expert order, then the shared expert's; n_tiles[0] and
+// n_tiles[1] are the counts before and with the shared ones.
 __global__ __launch_bounds__(1024) void k_mt_bucket(const int32_t *__restrict__ idx, int T, int K, int E,
                                                     int *__restrict__ pair_tok, int *__restrict__ pos_of,
-                                                    MtTile *__restrict__ tiles, int *__restrict__ n_tiles,
-                                                    int *__restrict__ work_gu, int *__restrict__ work_dn,
-                                                    int *__restrict__ n_work, int c_gu, int c_dn, int slots_gu,
-                                                    int slots_dn)
+                                                    MtTile *__restrict__ tiles, int *__restrict__ n_tiles)
 {
     __shared__ int cnt[1024], base[1024], cur[1024];
     __shared__ int wsa[16], wsb[16];
-    __shared__ int xfirst[NXCD + 1];
     const int tid = threadIdx.x;
     cnt[tid] = 0;
     cur[tid] = 0;
@@ -407,377 +296,807 @@ __global__ __launch_bounds__(1024) void k_mt_bucket(const int32_t *__restrict__ 
     const int nsh = (T + MT - 1) / MT;
     for (int i = tid; i < nsh; i += 1024) tiles[tt + i] = {E, P + i * MT, min(MT, T - i * MT), 0};
     for (int t = tid; t < T; t += 1024) pair_tok[P + t] = t;
-    const int N = tt + nsh;
-    if (tid == 0) *n_tiles = N;
-
-    // Work lists.  Segments of at most SEG consecutive tiles of one expert
-    // (the shared expert's after the routed ones) stay on one XCD, so the
-    // expert's weights are fetched into that L2 once per segment instead of
-    // once per tile, while a hot expert's segments still spread over the
-    // XCDs.  The segment starting at tile s0 goes to XCD floor(8 s0 / N),
-    // and XCD x holds tiles [A(x), A(x + 1)) with A(x) the first segment
-    // start >= ceil(x N / 8).  Per XCD, items run segment by segment,
-    // chunk-major: (tile s0 + i, chunk c) at (s0 - A(x)) C + c n + i.
-    // A(x + 1) - A(x) <= ceil(N / 8) + SEG, which the host sizes the lists
-    // for; writes beyond a list are dropped regardless.
-    cnt[tid] = xt;  // each expert's first tile (the counts are used up)
-    if (tid <= NXCD) xfirst[tid] = N;
-    __syncthreads();
-    auto xcd_of = [&](int start) { return min(NXCD - 1, (int)(((long long)start * NXCD) / N)); };
-    // tile q's segment: start and length.  Below tt the expert is the last
-    // one whose first tile is <= q (an empty expert shares its first tile
-    // with the next, so that one is never empty).
-    auto segment = [&](int q, int &start, int &len) {
-        int first = tt, ntiles = nsh;
-        if (q < tt) {
-            int lo = 0, hi = E - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (cnt[mid] <= q) lo = mid;
-                else hi = mid - 1;
-            }
-            first = cnt[lo];
-            ntiles = (cur[lo] + MT - 1) / MT;
-        }
-        start = first + (q - first) / SEG * SEG;
-        len = min(SEG, first + ntiles - start);
-    };
-    for (int q = tid; q < N; q += 1024) {
-        int start, len;
-        segment(q, start, len);
-        if (q == start) atomicMin(&xfirst[xcd_of(q)], q);
-    }
-    __syncthreads();
-    if (tid == 0)
-        for (int x = NXCD - 1; x >= 0; x--) xfirst[x] = min(xfirst[x], xfirst[x + 1]);
-    __syncthreads();
-    for (int q = tid; q < N; q += 1024) {
-        int start, len;
-        segment(q, start, len);
-        const int x = xcd_of(start), b = start - xfirst[x], i = q - start;
-        for (int cc = 0; cc < c_gu; cc++) {
-            const int j = b * c_gu + cc * len + i;
-            if (j < slots_gu) work_gu[x * slots_gu + j] = (q << 8) | cc;
-        }
-        for (int cc = 0; cc < c_dn; cc++) {
-            const int j = b * c_dn + cc * len + i;
-            if (j < slots_dn) work_dn[x * slots_dn + j] = (q << 8) | cc;
-        }
-    }
-    if (tid < NXCD) {
-        const int nx = xfirst[tid + 1] - xfirst[tid];
-        n_work[tid] = min(nx * c_gu, slots_gu);
-        n_work[NXCD + tid] = min(nx * c_dn, slots_dn);
+    if (tid == 0) {
+        n_tiles[0] = tt;
+        n_tiles[1] = tt + nsh;
     }
 }
 
 // ---------------------------------------------------------------------------
-// Gate/up: tile (M-tile, 128 rows).  Waves 0..3 own gate rows n0 + 32w +
-// [0, 32), waves 4..7 the same rows of up, one 32-row block per wave.  The
-// tile's 32 activation rows are staged per superblock (32 KB, hi and lo) in
-// two LDS buffers by LDS-direct loads one superblock ahead; each wave loads
-// its raw weight bytes one superblock ahead into registers and dequantises
-// them there.  One barrier per superblock; two workgroups (16 waves) per CU.
-// At the end the up waves pass their results through LDS to the gate waves
-// (same lane layout), which apply the SwiGLU (layer_ops.cu:214-220).
+// Raw superblock bytes of a lane: row r, half g of the superblock.
 // ---------------------------------------------------------------------------
 
-// Workgroups go to the 8 XCDs round-robin by linear id, and each XCD has its
-// own L2.  Workgroup L takes item L / 8 of XCD L % 8's list (k_mt_bucket);
-// false when that list is shorter.
-__device__ __forceinline__ bool xcd_item(const int *work, const int *n_work, int slots, int &tile, int &chunk)
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+template <int QT>
+struct Raw;
+
+template <>
+struct Raw<BREAD_QTYPE_Q4_K> {
+    static constexpr uint32_t BYTES = Q4K_BYTES;
+    uint4 hd, q[4];  // d, dmin, scales; the half's qs bytes
+};
+
+template <>
+struct Raw<BREAD_QTYPE_Q6_K> {
+    static constexpr uint32_t BYTES = Q6K_BYTES;
+    u32x4_a2 l[4], h[2];  // the half's ql and qh bytes
+    u32x2_a2 sc;          // its eight scales
+    uint32_t d;
+};
+
+__device__ __forceinline__ void raw_load(Raw<BREAD_QTYPE_Q4_K> &R, const uint8_t *p, uint32_t off, int g)
 {
-    const int L = (int)blockIdx.x;
-    const int x = L & (NXCD - 1), j = L / NXCD;
-    if (j >= n_work[x]) return false;
-    const int v = work[x * slots + j];
-    tile = v >> 8;
-    chunk = v & 255;
-    return true;
+    R.hd = *reinterpret_cast<const uint4 *>(p + off);
+    const uint32_t q = off + 16 + 64 * g;
+#pragma unroll
+    for (int i = 0; i < 4; i++) R.q[i] = *reinterpret_cast<const uint4 *>(p + (q + 16 * i));
 }
 
-__global__ __launch_bounds__(GU_WAVES * WAVE, 2) void k_mt_gateup(const MtArgs a)
+// Q6_K superblocks are 2-byte aligned; the loads say so (the target takes
+// unaligned vector loads) and stay inside the superblock.
+__device__ __forceinline__ void raw_load(Raw<BREAD_QTYPE_Q6_K> &R, const uint8_t *p, uint32_t off, int g)
 {
-    __shared__ uint4 sA[2][2][1024];  // [buffer][hi, lo][unit (s, g, n)]
-    __shared__ int stok[MT], sexp[MT];
-    int tile, chunk;
-    if (!xcd_item(a.work_gu, a.n_work, a.slots_gu, tile, chunk) || tile >= *a.n_tiles) return;
-    const MtTile tl = a.tiles[tile];
-    const bool sh = tl.e == a.E;
-    const int I = sh ? a.Ish : a.I;
-    const int n0 = chunk * GU_ROWS;
-    if (n0 >= I) return;
-    const int tid = threadIdx.x, w = wave_id(), lane = lane_id();
-    const bool up = w >= GU_WAVES / 2;
-    const int wr = up ? w - GU_WAVES / 2 : w;
-    const int g = lane >> 5, r = lane & 31;
-    if (tid < MT) {
-        const int tok = a.pair_tok[tl.p0 + min(tid, tl.nr - 1)];
-        stok[tid] = tok;
-        sexp[tid] = a.xexp[tok];
-    }
-    __syncthreads();
-
-    const int HU = a.H / 8, nsb = a.H / QK;
-    const uint64_t rb = (uint64_t)nsb * Q4K_BYTES;
-    const uint8_t *base = up ? (sh ? (const uint8_t *)a.L.up_shexp
-                                   : (const uint8_t *)a.L.up_exps + (uint64_t)tl.e * a.L.up_expert_bytes)
-                             : (sh ? (const uint8_t *)a.L.gate_shexp
-                                   : (const uint8_t *)a.L.gate_exps + (uint64_t)tl.e * a.L.gate_expert_bytes);
-    const int row0 = n0 + 32 * wr;
-    const uint8_t *wrow = base + (uint64_t)(row0 + r) * rb;
-    // unit (s, g, n) of a buffer: lane (n = r, g) of wave w stages s = w + 8i
-    const uint4 *ahi = a.xhi + (size_t)stok[r] * HU + 2 * w + g;
-    const uint4 *alo = a.xlo + (size_t)stok[r] * HU + 2 * w + g;
-
-    auto stage = [&](int sb, int st) {
+    const uint32_t l = off + 64 * g, h = off + 128 + 32 * g;
 #pragma unroll
-        for (int i = 0; i < 16 / GU_WAVES; i++) {
-            lds_load16(ahi + 32 * sb + 2 * GU_WAVES * i, &sA[st][0][64 * (w + GU_WAVES * i)]);
-            lds_load16(alo + 32 * sb + 2 * GU_WAVES * i, &sA[st][1][64 * (w + GU_WAVES * i)]);
-        }
-    };
-    auto load_b = [&](int sb, uint4 (&B)[5]) {
-        const uint8_t *p = wrow + (uint64_t)sb * Q4K_BYTES;
-        B[0] = ld_b128(p);
-#pragma unroll
-        for (int i = 0; i < 4; i++) B[1 + i] = ld_b128(p + 16 + 64 * g + 16 * i);
-    };
-    f32x16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.f;
-    // K-step s: activation fragments one step ahead of their MFMAs; the
-    // weight fragment from qs dword s%8 of pair 2g + s/8
-    auto ksteps = [&](int st, const uint4 (&B)[5], auto &&frag) {
-        uint4 xa[2][2];
-        xa[0][0] = sA[st][0][lane];
-        xa[0][1] = sA[st][1][lane];
-#pragma unroll
-        for (int s = 0; s < 16; s++) {
-            if (s + 1 < 16) {
-                xa[(s + 1) & 1][0] = sA[st][0][64 * (s + 1) + lane];
-                xa[(s + 1) & 1][1] = sA[st][1][64 * (s + 1) + lane];
-            }
-            __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of this step's work
-            const int pp = s >> 3, ds = s & 7;
-            const uint4 bw = frag(comp(B[1 + 2 * pp + (ds >> 2)], ds & 3), 2 * pp);
-            acc = mfma32(bw, xa[s & 1][0], acc);
-            acc = mfma32(bw, xa[s & 1][1], acc);
-        }
-    };
-    auto compute = [&](int st, const uint4 (&B)[5]) {
-        if (__builtin_amdgcn_ballot_w64(!q4k_pk_ok(B[0])) != 0 && lane == 0)
-            __hip_atomic_fetch_or(a.err, BREAD_DEV_ERR_RANGE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const Q4Pk pk = q4k_lane_pk(B[0], (uint32_t)g);
-        ksteps(st, B, [&](uint32_t v, int q) {
-            const uint32_t lo = v & 0x0F0F0F0Fu, hi = (v >> 4) & 0x0F0F0F0Fu;
-            uint4 r;
-            r.x = pk_w(__builtin_amdgcn_perm(MAGIC, lo, 0x07010700u), pk, q);
-            r.y = pk_w(__builtin_amdgcn_perm(MAGIC, lo, 0x07030702u), pk, q);
-            r.z = pk_w(__builtin_amdgcn_perm(MAGIC, hi, 0x07010700u), pk, q + 1);
-            r.w = pk_w(__builtin_amdgcn_perm(MAGIC, hi, 0x07030702u), pk, q + 1);
-            return r;
-        });
-    };
-
-    // Iteration k: wait for weights and activations of k (issued in
-    // iteration k-1), barrier (everyone is done with buffer (k+1)%2), issue
-    // k+1, compute k.
-    uint4 B0[5], B1[5];
-    load_b(0, B0);
-    stage(0, 0);
-    for (int sb = 0; sb < nsb; sb += 2) {
-        wait_vmcnt<0>();
-        __syncthreads();
-        if (sb + 1 < nsb) {
-            load_b(sb + 1, B1);
-            stage(sb + 1, 1);
-        }
-        compute(0, B0);
-        if (sb + 1 >= nsb) break;
-        wait_vmcnt<0>();
-        __syncthreads();
-        if (sb + 2 < nsb) {
-            load_b(sb + 2, B0);
-            stage(sb + 2, 0);
-        }
-        compute(1, B1);
-    }
-
-    const int e = sexp[r];
-    float *xch = reinterpret_cast<float *>(&sA[0][0][0]);  // [wave 0..3][16][64] up results
-    __syncthreads();
-    if (up) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) xch[(wr * 16 + i) * WAVE + lane] = ldexpf(acc[i], e);
-    }
-    __syncthreads();
-    if (!up && r < tl.nr) {
-        float *hp = a.h + (size_t)(tl.p0 + r) * a.Imax + row0 + 4 * g;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float4 o;
-            o.x = silu_mul(ldexpf(acc[4 * j + 0], e), xch[(wr * 16 + 4 * j + 0) * WAVE + lane]);
-            o.y = silu_mul(ldexpf(acc[4 * j + 1], e), xch[(wr * 16 + 4 * j + 1) * WAVE + lane]);
-            o.z = silu_mul(ldexpf(acc[4 * j + 2], e), xch[(wr * 16 + 4 * j + 2) * WAVE + lane]);
-            o.w = silu_mul(ldexpf(acc[4 * j + 3], e), xch[(wr * 16 + 4 * j + 3) * WAVE + lane]);
-            *reinterpret_cast<float4 *>(hp + 8 * j) = o;
-        }
-    }
+    for (int i = 0; i < 4; i++) R.l[i] = *reinterpret_cast<const u32x4_a2 *>(p + (l + 16 * i));
+    R.h[0] = *reinterpret_cast<const u32x4_a2 *>(p + h);
+    R.h[1] = *reinterpret_cast<const u32x4_a2 *>(p + (h + 16));
+    R.sc = *reinterpret_cast<const u32x2_a2 *>(p + (off + 192 + 8 * g));
+    R.d = *reinterpret_cast<const uint16_t *>(p + (off + 208));
 }
 
-// ---------------------------------------------------------------------------
-// Down: tile (M-tile, 512 output rows).  Wave w owns rows n0 + 64w + [0, 64)
-// as two 32-row blocks.  The tile's fp32 SwiGLU rows are read once, scaled
-// by a power of two per row and split into hi and lo fp16 parts in LDS (64 KB
-// for I = 512); each wave walks its (block, superblock) items loading the next
-// item's raw Q6_K bytes into registers while dequantising the current one.
-// ---------------------------------------------------------------------------
-
-__global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_mt_down(const MtArgs a)
+// D[32 tokens][32 rows] += X[32][16] * W[16][32]: D register i of lane (r, g)
+// holds token 8 (i / 4) + 4 g + i % 4 of row r.
+__device__ __forceinline__ f32x16 mfma32(const uint4 &x, const uint4 &w, f32x16 acc)
 {
-    __shared__ uint4 sA[2][(MAX_INTER / 8) * MT];  // [hi, lo][unit ((16b + t)*2 + g)*32 + n]
-    __shared__ int sexp[MT];
-    int tile, chunk;
-    if (!xcd_item(a.work_dn, a.n_work + NXCD, a.slots_dn, tile, chunk) || tile >= *a.n_tiles) return;
-    const MtTile tl = a.tiles[tile];
-    const bool sh = tl.e == a.E;
-    const int I = sh ? a.Ish : a.I;
-    const int n0 = chunk * DN_ROWS;
-    const int w = wave_id(), lane = lane_id();
-    const int g = lane >> 5, r = lane & 31;
-    const int nb = I / QK;
-    const uint64_t rbd = (uint64_t)nb * Q6K_BYTES;
-    const uint8_t *db = sh ? (const uint8_t *)a.L.down_shexp
-                           : (const uint8_t *)a.L.down_exps + (uint64_t)tl.e * a.L.down_expert_bytes;
-    const int row0 = n0 + 32 * DN_BLOCKS * w;
-    const int nblk = max(0, min(DN_BLOCKS, (a.H - row0) / 32));
-    const int items = nblk * nb;
-    auto item_ptr = [&](int it) {
-        return db + (uint64_t)(row0 + 32 * (it / nb) + r) * rbd + (uint64_t)(it % nb) * Q6K_BYTES;
-    };
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, x), __builtin_bit_cast(half8, w), acc, 0,
+                                                  0, 0);
+}
 
-    Q6Raw R0, R1;
-    if (items > 0) q6k_load(item_ptr(0), g, R0);
+__device__ __forceinline__ f32x16 zero16()
+{
+    f32x16 z;
+#pragma unroll
+    for (int i = 0; i < 16; i++) z[i] = 0.f;
+    return z;
+}
 
+__device__ __forceinline__ half2v h2_of(uint32_t v)
+{
+    return __builtin_bit_cast(half2v, v);
+}
+
+__device__ __forceinline__ uint32_t u_of(half2v v)
+{
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+__device__ __forceinline__ half2v dup(half2v v, int i)
+{
+    return half2v{v[i], v[i]};
+}
+
+__device__ __forceinline__ half2v pair(float a, float b)
+{
+    return half2v{(_Float16)a, (_Float16)b};
+}
+
+// Masks and magic numbers in registers: (v & mask) | magic is then one
+// three-operand instruction (with literals, which that form does not take,
+// the compiler makes two).
+struct Consts {
+    uint32_t lo, hi, q2, magic;  // 0x000F000F, 0x00F000F0, 0x00300030, fp16 1024 twice
+    uint32_t sca, scb;           // this lane's half: sc = (s & sca) | ((s0 >> 2) & scb), see Unit
+};
+
+__device__ __forceinline__ Consts consts(int g)
+{
+    Consts c;
+    asm("s_mov_b32 %0, 0x000F000F" : "=s"(c.lo));
+    asm("s_mov_b32 %0, 0x00F000F0" : "=s"(c.hi));
+    asm("s_mov_b32 %0, 0x00300030" : "=s"(c.q2));
+    asm("v_mov_b32 %0, 0x64006400" : "=v"(c.magic));
+    c.sca = g ? 0x0F0F0F0Fu : 0x3F3F3F3Fu;
+    c.scb = g ? 0x30303030u : 0u;
+    return c;
+}
+
+// Bytes I and J of v (small non-negative integers) as an fp16 pair.
+template <int I, int J>
+__device__ __forceinline__ half2v pair_u8(uint32_t v)
+{
+    return h2_of(__builtin_amdgcn_perm(0x64646464u, v, 0x07000700u | I | (J << 16))) - pair(1024.f, 1024.f);
+}
+
+// Operand maker of one unit (32 weight rows of one superblock): constants
+// from the superblock's header, then a step's eight weights; the scaling of
+// the sums.  prepare() sets bad when the superblock is outside the range that
+// fp16 weights can hold (checked where `flag`): Q4_K |d| >= 64 or |dmin| >=
+// 1024, Q6_K |d sc| >= 2047, or NaN.
+template <int QT>
+struct Unit;
+
+template <>
+struct Unit<BREAD_QTYPE_Q4_K> {
+    half2v sc[2], ns[2];
+
+    // Scales of groups 0, 1 and 2, 3: a pair each; odd groups meet 16 q (the
+    // nibble left in place).  fma(1024 + q, sc, -1024 sc) = sc q exactly.
+    __device__ __forceinline__ void prepare(const Raw<BREAD_QTYPE_Q4_K> &R, const Consts &C, int g, bool flag, bool &bad)
     {
-        // the tile's SwiGLU rows (fp32, by pair) scaled by a power of two per
-        // row and split into hi/lo fp16 in LDS: element group v (8 floats)
-        // of pair row p0 + n is LDS unit 64 (16 (v / 32) + v % 16) + 32 ((v /
-        // 16) % 2) + n.  Wave w takes rows 4w .. 4w+3, 16 lanes a row, groups
-        // gl + 16 k of the row.
-        const int rw = 4 * w + (lane >> 4), gl = lane & 15;
-        const int ng = I / 8;
-        const float *hr = a.h + (size_t)(tl.p0 + min(rw, tl.nr - 1)) * a.Imax;
-        float4 va[4], vb[4];
+        const uint32_t s0 = R.hd.y, s2 = R.hd.w;
+        if (flag) bad |= !(fabsf(h2f(R.hd.x)) < 64.f && fabsf(h2f(R.hd.x >> 16)) < 1024.f);
+        const uint32_t sc4 = ((g ? s2 : s0) & C.sca) | ((s0 >> 2) & C.scb);
+        const half2v p0 = pair_u8<0, 1>(sc4), p1 = pair_u8<2, 3>(sc4);
+        sc[0] = p0 * pair(1.f, 0.0625f);
+        sc[1] = p1 * pair(1.f, 0.0625f);
+        ns[0] = p0 * pair(-1024.f, -64.f);
+        ns[1] = p1 * pair(-1024.f, -64.f);
+    }
+
+    // tot += d * c - dmin * sum_j m_j * (sum of x over sub-block j): m_0..7
+    // against the hi and lo sums
+    __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q4_K> &R, const uint4 &sums, const f32x16 &c,
+                                        f32x16 &tot) const
+    {
+        const uint32_t s1 = R.hd.z, s2 = R.hd.w;
+        const uint32_t ml = s1 & 0x3F3F3F3Fu, mh = ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u);
+        const uint4 mv = make_uint4(u_of(pair_u8<0, 1>(ml)), u_of(pair_u8<2, 3>(ml)), u_of(pair_u8<0, 1>(mh)),
+                                    u_of(pair_u8<2, 3>(mh)));
+        const f32x16 pm = mfma32(sums, mv, zero16());
+        const float d = h2f(R.hd.x), dm = -32.f * h2f(R.hd.x >> 16);
+#pragma unroll
+        for (int i = 0; i < 16; i++) tot[i] = fmaf(c[i], d, tot[i]);
+#pragma unroll
+        for (int i = 0; i < 16; i++) tot[i] = fmaf(pm[i], dm, tot[i]);
+    }
+
+    template <bool X>
+    __device__ __forceinline__ void step(const Raw<BREAD_QTYPE_Q4_K> &R, const Consts &C, int s, uint4 &w, uint4 &) const
+    {
+        const int pp = s >> 3;
+        const uint32_t v = comp(R.q[s >> 2], s & 3), v8 = v >> 8;
+        const half2v se = dup(sc[pp], 0), so = dup(sc[pp], 1), ne = dup(ns[pp], 0), no = dup(ns[pp], 1);
+        w = make_uint4(u_of(__builtin_elementwise_fma(h2_of((v & C.lo) | C.magic), se, ne)),
+                       u_of(__builtin_elementwise_fma(h2_of((v8 & C.lo) | C.magic), se, ne)),
+                       u_of(__builtin_elementwise_fma(h2_of((v & C.hi) | C.magic), so, no)),
+                       u_of(__builtin_elementwise_fma(h2_of((v8 & C.hi) | C.magic), so, no)));
+    }
+};
+
+template <>
+struct Unit<BREAD_QTYPE_Q6_K> {
+    half2v sc[4];  // scales sc[8 g + 2 q], sc[8 g + 2 q + 1] of group q: elements 0..15 and 16..31
+
+    __device__ __forceinline__ void prepare(const Raw<BREAD_QTYPE_Q6_K> &R, const Consts &, int, bool flag, bool &bad)
+    {
+        const uint32_t a = R.sc[0] ^ 0x80808080u, b = R.sc[1] ^ 0x80808080u;  // sc + 128
+        const half2v k = pair(128.f, 128.f);
+        sc[0] = pair_u8<0, 1>(a) - k;
+        sc[1] = pair_u8<2, 3>(a) - k;
+        sc[2] = pair_u8<0, 1>(b) - k;
+        sc[3] = pair_u8<2, 3>(b) - k;
+        const float d = h2f(R.d);
+        if (flag && __builtin_amdgcn_ballot_w64(!(fabsf(d) < 15.9f)) != 0) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) bad |= !(fabsf(d * (float)sc[q >> 1][q & 1]) < 2047.f);
+        }
+    }
+
+    __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q6_K> &R, const uint4 &, const f32x16 &c,
+                                        f32x16 &tot) const
+    {
+        const float d = h2f(R.d);
+#pragma unroll
+        for (int i = 0; i < 16; i++) tot[i] = fmaf(c[i], d, tot[i]);
+    }
+
+    // w = fp16(sc (q - 32)); r (X): what that rounds off, 0 or +-1
+    template <bool X>
+    __device__ __forceinline__ void step(const Raw<BREAD_QTYPE_Q6_K> &R, const Consts &C, int s, uint4 &w, uint4 &r) const
+    {
+        const int pp = s >> 3, k = s & 7;
+        const uint32_t h = R.h[k >> 2][k & 3];
+        uint32_t wv[4], rv[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {  // group 2 pp + j / 2, bytes 0 and 2 (j even) or 1 and 3
+            const int q = 2 * pp + (j >> 1), lsh = 4 * pp + 8 * (j & 1), hsh = 8 * (j & 1) + 2 * q - 4;
+            const uint32_t l = R.l[(j >> 1) * 2 + (k >> 2)][k & 3] >> lsh;
+            const uint32_t hb = hsh >= 0 ? h >> hsh : h << -hsh;
+            const half2v v = h2_of((hb & C.q2) | ((l & C.lo) | C.magic)) - pair(1056.f, 1056.f);  // q - 32, exact
+            const half2v se = dup(sc[q], k >> 2), p = v * se;
+            wv[j] = u_of(p);
+            rv[j] = X ? u_of(__builtin_elementwise_fma(v, se, -p)) : 0;
+        }
+        w = make_uint4(wv[0], wv[1], wv[2], wv[3]);
+        r = make_uint4(rv[0], rv[1], rv[2], rv[3]);
+    }
+};
+
+// silu(g) * u (layer_ops.cu:214-220): exp from the hardware's exp2 with the
+// rounding of g log2(e) added back, the quotient by Newton steps on the
+// hardware reciprocal; exact division where that could overflow.
+__device__ __forceinline__ float swiglu(float g, float u)
+{
+    const float t = -1.44269504088896f * g;
+    const float lo = fmaf(-1.44269504088896f, g, -t) + g * -1.925963033500e-8f;  // t's rounding, log2(e)'s
+    const float e = __builtin_amdgcn_exp2f(t);
+    const float den = 1.0f + (fabsf(t) < 128.f ? fmaf(e, 0.693147180559945f * lo, e) : e);
+    float q = __builtin_amdgcn_rcpf(den);
+    q = fmaf(fmaf(-den, q, 1.0f), q, q);
+    float v = g * q;
+    v = fmaf(fmaf(-den, v, g), q, v);
+    return (den < 1e30f ? v : g / den) * u;
+}
+
+struct GgArgs {
+    const uint8_t *w0, *w1;    // routed gate and up (or down), expert e at + e * stride
+    uint64_t st0, st1;
+    const uint8_t *sw0, *sw1;  // the shared expert's
+    uint32_t *err;
+    const uint4 *xop, *xsum;   // prepared activations by token
+    const int *xexp;
+    const int *pair_tok;
+    const MtTile *tiles;
+    const int *n_tiles;
+    float *h;                  // SwiGLU rows by tile [tiles][MT][hstride]
+    float *eo;                 // expert outputs by pair [pairs][H]
+    int E, nsb, rows;          // superblocks of the contraction, rows per expert
+    int hstride;
+    int sel;                   // 0: all tiles, 1: routed, 2: shared
+    int flag;                  // report superblocks outside the fp16 range
+};
+
+#define CONST_AS __attribute__((address_space(4)))  // read by scalar loads
+
+// The items of a workgroup: (tile, chunk of rows), the chunks of a tile in
+// sequence, C a tile.  Workgroups go to the 8 XCDs round-robin by linear id and
+// each XCD has its own L2, so XCD L % 8 takes a contiguous eighth, where a
+// tile's chunks share its activations and an expert's tiles its weights; its
+// workgroups take turns.
+struct GgItems {
+    const MtTile CONST_AS *tiles;
+    int lo, N, per, j, i, C;
+    int tile, chunk, e, p0, nr;  // the current item
+
+    __device__ __forceinline__ GgItems(const GgArgs &a, int chunks)
+    {
+        const int CONST_AS *n = (const int CONST_AS *)a.n_tiles;
+        tiles = (const MtTile CONST_AS *)a.tiles;
+        C = chunks;
+        lo = a.sel == 2 ? n[0] : 0;
+        N = ((a.sel == 1 ? n[0] : n[1]) - lo) * C;
+        per = (N + NXCD - 1) / NXCD;
+        j = (int)blockIdx.x / NXCD - (int)gridDim.x / NXCD;
+        i = ((int)blockIdx.x % NXCD) * per;
+    }
+    // the next item, false (and the last one kept) past the end
+    __device__ __forceinline__ bool next()
+    {
+        j += (int)gridDim.x / NXCD;
+        if (j >= per || i + j >= N) return false;
+        tile = uniform(lo + (i + j) / C);
+        chunk = uniform((i + j) % C);
+        e = uniform(tiles[tile].e);
+        p0 = uniform(tiles[tile].p0);
+        nr = uniform(tiles[tile].nr);
+        return true;
+    }
+};
+
+__device__ __forceinline__ void lds_load16(const void *src, void *lds_wave_base)
+{
+    __builtin_amdgcn_global_load_lds(src, lds_wave_base, 16, 0, 0);
+}
+
+// A barrier that publishes the waves' LDS writes and leaves global loads in
+// flight (__syncthreads would wait for every one of them).
+__device__ __forceinline__ void gg_bar()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt at their maxima
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// s_waitcnt on the vector memory counter only (gfx9 encoding).
+template <int N>
+__device__ __forceinline__ void wait_vm()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Units u = 2 s + g, s = 0 .. 7, of row r in LDS rows of 32 units (16 hi, 16
+// lo; half a superblock) or 64 (32 hi, 32 lo): unit u of token n is at u ^ (n
+// % 16), so that a read of one unit of 16 tokens covers the banks.  The
+// address is made anew each time: the compiler would keep eight of them in
+// registers for the whole kernel.
+struct XRead {
+    const char *p;
+    uint32_t a;
+    __device__ __forceinline__ XRead(const uint4 *row, int r, int g)
+    {
+        p = reinterpret_cast<const char *>(row);
+        a = (uint32_t)(16 * (g ^ (r & 15)));
+        asm volatile("" : "+v"(a));
+    }
+    __device__ __forceinline__ uint4 operator()(int s, uint32_t off) const
+    {
+        return *reinterpret_cast<const uint4 *>(p + ((a ^ (uint32_t)(32 * (s & 7))) + off));
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Gate/up: workgroup of 4 waves per (tile, 128 rows); a wave owns 32 gate
+// rows and the same 32 up rows, so each activation fragment read from LDS
+// meets 64 weight rows and the SwiGLU needs no exchange.
+// The workgroups are persistent: the last superblock of an item requests the
+// first one of the next.
+//
+// Everything comes by direct-to-LDS loads whose adjacent lanes read adjacent
+// memory: a load whose lanes are 64 rows costs the address unit a cycle a
+// lane, and with the weights loaded so (16 bytes of a row a lane) issuing a
+// superblock's loads took 2,500-5,000 cycles of an iteration of 8,500.  Weights: a wave's 2 x 32 rows of a superblock (9 KB) into a buffer
+// of its own, moved to registers when the superblock begins, which frees the
+// buffer for the next one.  Activations: half a superblock of the tile's 32
+// rows (16 KB) into one of two buffers, a half ahead.  A barrier each half;
+// 70 KB of LDS, two workgroups a CU.
+// Q6_K gate or up (no reference GPU layout) loads its weights straight into
+// registers: its 210-byte superblocks are 2-byte aligned.
+//
+// Measured on MI355X (hidden 2048, intermediate 512, 256 experts, top 8), the
+// kernel that dequantised into fp16 d sc q - dmin m operands with a lane a
+// weight row / this one: 64 tokens (Zipf) 36 / 28 us, 512 tokens 136 / 110 us,
+// 2048 tokens 321 / 253 us.  A superblock (2 x 32 MFMA a wave, 8 waves a CU)
+// takes 6,500 cycles against 4,200 of the matrix pipe alone; half the rest is
+// issuing the direct-to-LDS loads, and an item's prologue and SwiGLU add
+// 6,000.  At 512 tokens (16 pairs an expert) half of a tile's rows are empty.
+// ---------------------------------------------------------------------------
+
+constexpr int W_CHUNKS = 32 * Q4K_BYTES / 16;  // 16-byte pieces of a matrix's superblock rows of a wave
+constexpr int W_LOADS = (W_CHUNKS + WAVE - 1) / WAVE;
+constexpr int W_BUF = W_LOADS * WAVE;  // the last load's idle lanes repeat the last piece
+
+template <int Q0, int Q1>
+__global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
+{
+    constexpr int Q4 = BREAD_QTYPE_Q4_K;
+    constexpr bool X0 = Q0 != Q4, X1 = Q1 != Q4, SUMS = Q0 == Q4 || Q1 == Q4;
+    // a variable for each buffer: a read of one that a direct-to-LDS load may
+    // write waits for all such loads
+    __shared__ uint4 sA0[MT][32], sA1[MT][32], sS[MT][2];
+    __shared__ uint4 sW[GG_WAVES][(Q0 == Q4) + (Q1 == Q4) ? (Q0 == Q4) + (Q1 == Q4) : 1][W_BUF];
+    __shared__ int sexp[2][MT];
+    const int tid = (int)threadIdx.x, w = wave_id(), lane = lane_id();
+    const int g = lane >> 5, r = lane & 31;
+    GgItems it(a, a.rows / GU_ROWS);
+    if (!it.next()) return;
+    const uint32_t rb0 = (uint32_t)a.nsb * Raw<Q0>::BYTES, rb1 = (uint32_t)a.nsb * Raw<Q1>::BYTES;
+    // the item's matrices, from the wave's first row (n0, n1: the next item's)
+    const uint8_t *m0, *m1, *n0, *n1;
+    auto matrices = [&](const uint8_t *&p, const uint8_t *&q) __attribute__((always_inline)) {
+        const uint32_t row0 = (uint32_t)(it.chunk * GU_ROWS + 32 * w);
+        p = (it.e == a.E ? a.sw0 : a.w0 + (uint64_t)it.e * a.st0) + (uint64_t)row0 * rb0;
+        q = (it.e == a.E ? a.sw1 : a.w1 + (uint64_t)it.e * a.st1) + (uint64_t)row0 * rb1;
+    };
+
+    // 16-byte piece c of a matrix's superblock rows: row c / 9, piece c % 9
+    uint32_t wo[W_LOADS];
+#pragma unroll
+    for (int j = 0; j < W_LOADS; j++) {
+        const uint32_t c = (uint32_t)min(64 * j + lane, W_CHUNKS - 1);
+        wo[j] = (c / 9) * ((uint32_t)a.nsb * Q4K_BYTES) + (c % 9) * 16;
+    }
+    auto stage_m = [&](const uint8_t *m, int sb, uint4 (&buf)[W_BUF]) __attribute__((always_inline)) {
+        const uint8_t *p = m + (uint32_t)sb * Q4K_BYTES;
+#pragma unroll
+        for (int j = 0; j < W_LOADS; j++)
+            lds_load16(p + wo[j], &buf[64 * j]);
+    };
+    Raw<Q0> R0;
+    Raw<Q1> R1;
+    constexpr int S1 = Q0 == Q4 ? 1 : 0;  // the up matrix's buffer
+    auto stage_w = [&](const uint8_t *p, const uint8_t *q, int sb) __attribute__((always_inline)) {
+        if constexpr (Q0 == Q4) stage_m(p, sb, sW[w][0]);
+        if constexpr (Q1 == Q4) stage_m(q, sb, sW[w][S1]);
+    };
+    // the wave's weights of superblock sb into registers: lane (r, g)
+    auto take_q4 = [&](Raw<Q4> &R, const uint4 (&buf)[W_BUF]) __attribute__((always_inline)) {
+        R.hd = buf[9 * r];
+#pragma unroll
+        for (int i = 0; i < 4; i++) R.q[i] = buf[9 * r + 1 + 4 * g + i];
+    };
+    auto take_w = [&](int sb) __attribute__((always_inline)) {
+        if constexpr (Q0 == Q4) take_q4(R0, sW[w][0]);
+        else raw_load(R0, m0 + (uint32_t)sb * Raw<Q0>::BYTES, (uint32_t)r * rb0, g);
+        if constexpr (Q1 == Q4) take_q4(R1, sW[w][S1]);
+        else raw_load(R1, m1 + (uint32_t)sb * Raw<Q1>::BYTES, (uint32_t)r * rb1, g);
+    };
+    constexpr int NW = W_LOADS * ((Q0 == Q4) + (Q1 == Q4));  // loads of stage_w
+
+    // Tokens 2 q and 2 q + 1, q = w, w + 4, ...: an instruction brings half
+    // a superblock of both, 16 hi and 16 lo units each (past nr the last
+    // token: its results are not stored).  Every wave brings the sums: a
+    // branch would blur the wait counts.
+    constexpr int NT = MT / (2 * GG_WAVES);
+    int tok[NT], tsum;
+    const char *xt[NT];
+    const uint4 *xs;
+    auto tokens = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NT; i++)
+            tok[i] = a.pair_tok[it.p0 + min(2 * (w + GG_WAVES * i) + (lane >> 5), it.nr - 1)];
+        tsum = a.pair_tok[it.p0 + min(lane >> 1, it.nr - 1)];
+    };
+    auto pointers = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NT; i++) {
+            const int n = 2 * (w + GG_WAVES * i) + (lane >> 5), u = lane & 31;
+            xt[i] = reinterpret_cast<const char *>(a.xop + (size_t)tok[i] * a.nsb * 64) + 512 * (u >> 4) +
+                    16 * ((u ^ n) & 15);
+        }
+        xs = a.xsum + (size_t)tsum * a.nsb * 2 + (lane & 1);
+    };
+    auto stage_x = [&](int sb, int pp, uint4 (&buf)[MT][32]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NT; i++)
+            lds_load16(xt[i] + (sb * 1024 + pp * 256), &buf[2 * (w + GG_WAVES * i)][0]);
+    };
+
+    const Consts C = consts(g);
+    f32x16 t0 = zero16(), t1 = zero16(), c0, c1;
+    Unit<Q0> U0;
+    Unit<Q1> U1;
+    bool bad = false;
+    // steps 8 pp .. 8 pp + 7 of the superblock in R0, R1
+    auto compute = [&](const uint4 (&sA)[MT][32], int pp) __attribute__((always_inline)) {
+        const XRead x(sA[r], r, g);
+        uint4 xh = x(0, 0), xl = x(0, 256), nh, nl;
+        uint4 w0, w1, r0, r1, v0, v1, q0, q1;
+        U0.template step<X0>(R0, C, 8 * pp, w0, r0);
+        U1.template step<X1>(R1, C, 8 * pp, w1, r1);
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            if (s < 7) {
+                nh = x(s + 1, 0);
+                nl = x(s + 1, 256);
+            }
+            c0 = mfma32(xh, w0, c0);
+            c1 = mfma32(xh, w1, c1);
+            c0 = mfma32(xl, w0, c0);
+            c1 = mfma32(xl, w1, c1);
+            if (X0) c0 = mfma32(xh, r0, c0);
+            if (X1) c1 = mfma32(xh, r1, c1);
+            if (s < 7) {
+                U0.template step<X0>(R0, C, 8 * pp + s + 1, v0, q0);
+                U1.template step<X1>(R1, C, 8 * pp + s + 1, v1, q1);
+            }
+            // an MFMA, then VALU: the next step's operands are made under
+            // this one's products
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, X0 || X1 ? 14 : 5, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            xh = nh;
+            xl = nl;
+            w0 = v0;
+            w1 = v1;
+            r0 = q0;
+            r1 = q1;
+        }
+    };
+
+    matrices(m0, m1);
+    tokens();
+    pointers();
+    stage_x(0, 0, sA0);
+    stage_w(m0, m1, 0);
+    bool first = true;
+    for (int turn = 0;; turn ^= 1, first = false) {
+        const int tile = it.tile, nr = it.nr, row0 = it.chunk * GU_ROWS + 32 * w;
+        const int ex_tok = a.pair_tok[it.p0 + min(tid & (MT - 1), nr - 1)];
+        const bool more = it.next();
+        matrices(n0, n1);
+        tokens();
+        if (tid < MT) sexp[turn][tid] = a.xexp[ex_tok];
+        t0 = t1 = zero16();
+        for (int sb = 0; sb < a.nsb; sb++) {
+            // First half: activations and weights have landed.  The sums and
+            // the second half's activations go out, then (behind them, so
+            // that the next wait can leave them in flight) the next
+            // superblock's weights, at the end the next item's first ones.
+            const bool last = sb + 1 == a.nsb;
+            if (sb == 0 && !first) wait_vm<16>();  // the last item's 16 stores
+            else wait_vm<0>();
+            gg_bar();
+            take_w(sb);
+            if (SUMS) lds_load16(xs + 2 * sb, &sS[0][0]);
+            stage_x(sb, 1, sA1);
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's buffer is read
+            __builtin_amdgcn_sched_barrier(0);
+            stage_w(last ? n0 : m0, last ? n1 : m1, last ? 0 : sb + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            U0.prepare(R0, C, g, a.flag != 0, bad);
+            U1.prepare(R1, C, g, a.flag != 0, bad);
+            c0 = c1 = zero16();
+            compute(sA0, 0);
+            // second half
+            wait_vm<NW>();
+            gg_bar();
+            if (last) pointers();
+            stage_x(last ? 0 : sb + 1, 0, sA0);
+            compute(sA1, 1);
+            uint4 sums = make_uint4(0, 0, 0, 0);
+            if (SUMS) sums = sS[r][g];
+            U0.add(R0, sums, c0, t0);
+            U1.add(R1, sums, c1, t1);
+        }
+        // SwiGLU, stored in operand order: row c of a superblock at its
+        // unit's place (unit_base), for k_down_gg's loads
+        const int c = (row0 + r) & (QK - 1);
+        const int u = 2 * (8 * ((c >> 6) & 1) + ((c >> 2) & 7)) + (c >> 7);
+        const uint32_t col = (uint32_t)(((row0 + r) & ~(QK - 1)) + 8 * u + 4 * ((c >> 5) & 1) + 2 * (c & 1) + ((c >> 1) & 1));
+        // rows past nr fall outside the buffer's range: every lane issues all
+        // 16 stores, which the next item's first wait leaves in flight
+        const __amdgpu_buffer_rsrc_t hb = rsrc(a.h + (size_t)tile * MT * a.hstride, (uint32_t)(nr * a.hstride * 4));
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int n = 8 * (i >> 2) + 4 * g + (i & 3);
+            const int ex = sexp[turn][n];
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, swiglu(ldexpf(t0[i], ex), ldexpf(t1[i], ex))),
+                                                  hb, 4 * (uint32_t)(n * a.hstride) + 4 * col, 0, 0);
+        }
+        if (!more) break;
+        m0 = n0;
+        m1 = n1;
+    }
+    wait_vm<0>();  // (the loads past the end)
+    if (a.flag && __builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0)
+        __hip_atomic_fetch_or(a.err, BREAD_DEV_ERR_RANGE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---------------------------------------------------------------------------
+// Down: workgroup of 8 waves per (tile, 512 output rows), a wave two 32-row
+// blocks.  The tile's fp32 SwiGLU rows (operand order) are read once, scaled
+// by a power of two per row and split into hi and lo fp16 parts in LDS (64 KB
+// for intermediate 512).  A unit is a block's 32 rows of one superblock: its
+// bytes come by direct-to-LDS loads of adjacent 16-byte pieces into the wave's
+// buffer, from there into registers when the unit begins, which frees the
+// buffer for the next one (loads of 16 bytes of a row a lane, 2-byte aligned,
+// took the address unit a cycle a lane).  The next item's SwiGLU rows and
+// first unit are requested while the last units run.
+// Measured as above, a lane a weight row / this: 64 tokens 23 / 23 us, 512
+// tokens 98 / 95 us, 2048 tokens 221 / 230 us (exact integer operands, a third
+// of the error).  A unit of 32 MFMA takes 3,500 cycles in its steps (VALU: a
+// Q6_K operand is some 20 instructions), 2,000 in its loads and its move to
+// registers.
+// ---------------------------------------------------------------------------
+
+// 16-byte pieces a row of a unit takes in the wave's buffer: a Q4_K superblock
+// is 9; a Q6_K one lies in the 14 aligned pieces from the one that holds its
+// first byte (inside the expert, whose start and size are 16-byte aligned),
+// and a 15th, unused, spreads the rows over the banks.
+template <int QT>
+constexpr int ROW_CH = QT == BREAD_QTYPE_Q4_K ? 9 : 15;
+template <int QT>
+constexpr int UNIT_LD = (32 * ROW_CH<QT> + WAVE - 1) / WAVE;  // loads of a unit
+
+// Lane (r, g)'s raw bytes from its buffer row; o: where the superblock starts
+// in it (even, below 16).
+__device__ __forceinline__ void take_unit(Raw<BREAD_QTYPE_Q4_K> &R, const uint4 *row, int g, uint32_t)
+{
+    R.hd = row[0];
+#pragma unroll
+    for (int i = 0; i < 4; i++) R.q[i] = row[1 + 4 * g + i];
+}
+
+__device__ __forceinline__ void take_unit(Raw<BREAD_QTYPE_Q6_K> &R, const uint4 *row, int g, uint32_t o)
+{
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(row) + (o >> 2);
+    const uint32_t sh = o & 2;
+    auto take = [&](const uint32_t *q, int n, auto &&put) __attribute__((always_inline)) {
+        uint32_t a = q[0];
+#pragma unroll
+        for (int i = 0; i < n; i++) {
+            const uint32_t b = q[i + 1];
+            put(i, __builtin_amdgcn_alignbyte(b, a, sh));
+            a = b;
+        }
+    };
+    take(p + 16 * g, 16, [&](int i, uint32_t v) { R.l[i >> 2][i & 3] = v; });
+    take(p + 32 + 8 * g, 8, [&](int i, uint32_t v) { R.h[i >> 2][i & 3] = v; });
+    take(p + 48 + 2 * g, 2, [&](int i, uint32_t v) { R.sc[i] = v; });
+    R.d = p[52] >> (8 * sh);
+}
+
+template <int QT, bool X>
+__global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
+{
+    constexpr int Q4 = BREAD_QTYPE_Q4_K;
+    constexpr bool X0 = X && QT != Q4;
+    constexpr int NB = MAX_INTER / QK;
+    __shared__ uint4 sA[NB][MT][64];
+    __shared__ uint32_t sS[QT == Q4 ? NB : 1][MT][2][4];  // sums: hi, lo of eight
+    __shared__ uint4 sW[DN_WAVES][UNIT_LD<QT> * WAVE];
+    __shared__ int sexp[MT];
+    const int tid = (int)threadIdx.x, w = wave_id(), lane = lane_id();
+    const int g = lane >> 5, r = lane & 31;
+    GgItems it(a, (a.rows + DN_ROWS - 1) / DN_ROWS);
+    if (!it.next()) return;
+    const int nb = a.nsb;
+    const uint32_t rb = (uint32_t)nb * Raw<QT>::BYTES;
+    // the item's matrix from the wave's first row; blocks past the end
+    // repeat the last one and are not stored
+    auto matrix = [&]() __attribute__((always_inline)) {
+        return (it.e == a.E ? a.sw0 : a.w0 + (uint64_t)it.e * a.st0);
+    };
+    auto block_row = [&](int chunk, int blk) __attribute__((always_inline)) {
+        return chunk * DN_ROWS + 32 * (DN_BLOCKS * w + blk);
+    };
+    // piece 64 j + lane of a unit: its row's offset and the piece's
+    uint32_t ro[UNIT_LD<QT>], po[UNIT_LD<QT>];
+#pragma unroll
+    for (int j = 0; j < UNIT_LD<QT>; j++) {
+        const uint32_t c = (uint32_t)min(64 * j + lane, 32 * ROW_CH<QT> - 1);
+        ro[j] = c / ROW_CH<QT> * rb;
+        po[j] = 16 * min(c % ROW_CH<QT>, (uint32_t)(QT == Q4 ? 8 : 13));
+    }
+    // unit u: block u / nb, superblock u % nb
+    auto stage_w = [&](const uint8_t *m, int chunk, int u) __attribute__((always_inline)) {
+        const int blk = nb == 2 ? u >> 1 : u, b = u - blk * nb;
+        const uint8_t *p = m + (uint64_t)(uint32_t)min(block_row(chunk, blk), a.rows - 32) * rb;
+#pragma unroll
+        for (int j = 0; j < UNIT_LD<QT>; j++)
+            lds_load16(p + (((ro[j] + (uint32_t)b * Raw<QT>::BYTES) & ~15u) + po[j]), &sW[w][64 * j]);
+    };
+    // 16 threads a token, each the units q + 16 k of its superblocks
+    const int hn = tid >> 4, hq = tid & 15;
+    float4 va[2 * NB], vb[2 * NB];
+    auto load_h = [&]() __attribute__((always_inline)) {
+        const float *hr = a.h + ((size_t)it.tile * MT + min(hn, it.nr - 1)) * a.hstride + 8 * hq;
+#pragma unroll
+        for (int k = 0; k < 2 * NB; k++) {
+            va[k] = vb[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (k < 2 * nb) {
+                va[k] = *reinterpret_cast<const float4 *>(hr + 128 * k);
+                vb[k] = *reinterpret_cast<const float4 *>(hr + 128 * k + 4);
+            }
+        }
+    };
+    auto split_h = [&]() __attribute__((always_inline)) {
         float mx = 0.f;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int v = gl + 16 * k;
-            va[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-            vb[k] = va[k];
-            if (v < ng) {
-                va[k] = *reinterpret_cast<const float4 *>(hr + 8 * v);
-                vb[k] = *reinterpret_cast<const float4 *>(hr + 8 * v + 4);
-            }
-            mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(fabsf(va[k].x), fabsf(va[k].y)), fmaxf(fabsf(va[k].z), fabsf(va[k].w))),
-                                 fmaxf(fmaxf(fabsf(vb[k].x), fabsf(vb[k].y)), fmaxf(fabsf(vb[k].z), fabsf(vb[k].w)))));
+        for (int k = 0; k < 2 * NB; k++) {
+            const float4 x = va[k], y = vb[k];
+            mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))),
+                                 fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w)))));
         }
-        mx = fmaxf(mx, dpp_f<0xB1>(mx));   // the 16 lanes of the row
+        mx = fmaxf(mx, dpp_f<0xB1>(mx));  // the token's 16 lanes
         mx = fmaxf(mx, dpp_f<0x4E>(mx));
         mx = fmaxf(mx, dpp_f<0x141>(mx));
         mx = fmaxf(mx, dpp_f<0x140>(mx));
-        const int e = row_exp(mx);
-        if (gl == 0) sexp[rw] = e;
+        const int ex = row_exp(mx);
+        if (hq == 0) sexp[hn] = ex;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int v = gl + 16 * k;
-            if (v < ng) {
-                const float x8[8] = {va[k].x, va[k].y, va[k].z, va[k].w, vb[k].x, vb[k].y, vb[k].z, vb[k].w};
-                uint4 hi, lo;
-                split8(x8, e, hi, lo);
-                const int u = 64 * (16 * (v >> 5) + (v & 15)) + 32 * ((v >> 4) & 1) + rw;
-                sA[0][u] = hi;
-                sA[1][u] = lo;
-            }
-        }
-    }
-    __syncthreads();
-
-    f32x16 acc;
-#pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.f;
-    auto compute = [&](int it, const Q6Raw &R) {
-        const uint32_t sh8 = (uint32_t)(reinterpret_cast<uintptr_t>(item_ptr(it)) & 3u);
-        const uint32_t qw[17] = {R.ql[0].x, R.ql[0].y, R.ql[0].z, R.ql[0].w, R.ql[1].x, R.ql[1].y,
-                                 R.ql[1].z, R.ql[1].w, R.ql[2].x, R.ql[2].y, R.ql[2].z, R.ql[2].w,
-                                 R.ql[3].x, R.ql[3].y, R.ql[3].z, R.ql[3].w, R.ql4};
-        const uint32_t hw[9] = {R.qh[0].x, R.qh[0].y, R.qh[0].z, R.qh[0].w, R.qh[1].x,
-                                R.qh[1].y, R.qh[1].z, R.qh[1].w, R.qh2};
-        // sc[8g .. 8g+3] and sc[8g+4 .. 8g+7]; g is per lane, so the words
-        // are picked by selects rather than by an indexed array
-        const uint32_t w0 = g ? R.sc.z : R.sc.x, w1 = g ? R.sc.w : R.sc.y, w2 = g ? R.sc1 : R.sc.z;
-        const uint32_t s0 = __builtin_amdgcn_alignbyte(w1, w0, sh8);
-        const uint32_t s1 = __builtin_amdgcn_alignbyte(w2, w1, sh8);
-        const float d = h2f(R.sc1 >> (8 * sh8));
-        const int b = it % nb;
-        bool bad = false;  // |d sc| * 32 beyond fp16's range
-        // K-steps t and t + 8 use the same ql bytes (low and high nibbles)
-        // and the same qh bytes (bits 2(t/4) and 2(t/4) + 4)
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            const uint32_t l0 = __builtin_amdgcn_alignbyte(qw[2 * t + 1], qw[2 * t], sh8);
-            const uint32_t l1 = __builtin_amdgcn_alignbyte(qw[2 * t + 2], qw[2 * t + 1], sh8);
-            const uint32_t h0 = __builtin_amdgcn_alignbyte(hw[2 * (t & 3) + 1], hw[2 * (t & 3)], sh8);
-            const uint32_t h1 = __builtin_amdgcn_alignbyte(hw[2 * (t & 3) + 2], hw[2 * (t & 3) + 1], sh8);
-#pragma unroll
-            for (int hi = 0; hi < 2; hi++) {
-                const int tt = t + 8 * hi;
-                const int hs = 2 * (tt >> 2);
-                const uint32_t scw = hi ? s1 : s0;
-                const float ds = d * (float)(int8_t)byte_of(scw, (uint32_t)((t >> 1) & 3));
-                const float c = -1056.f * ds;
-                bad |= !(fabsf(ds) < 2047.f);
-                const uint32_t n0v = (hi ? l0 >> 4 : l0) & 0x0F0F0F0Fu;
-                const uint32_t n1v = (hi ? l1 >> 4 : l1) & 0x0F0F0F0Fu;
-                const uint32_t q0 = n0v | (((h0 >> hs) & 0x03030303u) << 4);
-                const uint32_t q1 = n1v | (((h1 >> hs) & 0x03030303u) << 4);
-                uint4 bw;
-                bytes_to_w(q0, ds, c, bw.x, bw.y);
-                bytes_to_w(q1, ds, c, bw.z, bw.w);
-                const int unit = (16 * b + tt) * 64 + lane;
-                acc = mfma32(bw, sA[0][unit], acc);
-                acc = mfma32(bw, sA[1][unit], acc);
-            }
-        }
-        if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0)
-            __hip_atomic_fetch_or(a.err, BREAD_DEV_ERR_RANGE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (b == nb - 1) {
-            if (r < tl.nr) {
-                const int e = sexp[r];
-                float *op = a.eo + (size_t)(tl.p0 + r) * a.H + row0 + 32 * (it / nb) + 4 * g;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    float4 o;
-                    o.x = ldexpf(acc[4 * j + 0], e);
-                    o.y = ldexpf(acc[4 * j + 1], e);
-                    o.z = ldexpf(acc[4 * j + 2], e);
-                    o.w = ldexpf(acc[4 * j + 3], e);
-                    *reinterpret_cast<float4 *>(op + 8 * j) = o;
+        for (int k = 0; k < 2 * NB; k++) {
+            if (k >= 2 * nb) continue;
+            const int b = k >> 1, u = hq + 16 * (k & 1);
+            uint4 hi, lo;
+            split_unit_op(va[k], vb[k], ex, hi, lo);
+            sA[b][hn][u ^ (hn & 15)] = hi;
+            sA[b][hn][32 + (u ^ (hn & 15))] = lo;
+            if (QT == Q4) {
+                // sub-blocks 4 g + 2 (k & 1) (x) and the next (y), g = hq & 1:
+                // sums over the half's lanes
+                const float4 x = va[k], y = vb[k];
+                float sx = ldexpf((x.x + x.y) + (x.z + x.w), -ex - 5);
+                float sy = ldexpf((y.x + y.y) + (y.z + y.w), -ex - 5);
+                sx = xor_add(xor_add(xor_add(sx, 2), 4), 8);
+                sy = xor_add(xor_add(xor_add(sy, 2), 4), 8);
+                if (hq < 2) {
+                    uint32_t h2, l2;
+                    split2(sx, sy, h2, l2);
+                    sS[b][hn][0][2 * hq + (k & 1)] = h2;
+                    sS[b][hn][1][2 * hq + (k & 1)] = l2;
                 }
             }
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[i] = 0.f;
         }
     };
 
-    for (int it = 0; it < items; it += 2) {
-        if (it + 1 < items) q6k_load(item_ptr(it + 1), g, R1);
-        compute(it, R0);
-        if (it + 1 >= items) break;
-        if (it + 2 < items) q6k_load(item_ptr(it + 2), g, R0);
-        compute(it + 1, R1);
+    const Consts C = consts(g);
+    f32x16 t = zero16();
+    Raw<QT> R;
+    Unit<QT> U;
+    bool bad = false;
+    const uint8_t *m = matrix();
+    bool stores = false;  // the last unit stored
+    load_h();
+    stage_w(m, it.chunk, 0);
+    for (;;) {
+        const int chunk = it.chunk, p0 = it.p0, nr = it.nr;
+        const uint8_t *mc = m;
+        split_h();
+        gg_bar();
+        const bool more = it.next();
+        m = matrix();
+        for (int u = 0; u < DN_BLOCKS * nb; u++) {
+            const int blk = nb == 2 ? u >> 1 : u, b = u - blk * nb;
+            const int row0 = block_row(chunk, blk);
+            if (stores) wait_vm<16>();  // the last unit's 16 stores
+            else wait_vm<0>();
+            take_unit(R, &sW[w][r * ROW_CH<QT>], g, ((uint32_t)r * rb + (uint32_t)b * Raw<QT>::BYTES) & 15u);
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the wave's buffer is read
+            __builtin_amdgcn_sched_barrier(0);
+            const bool last = u + 1 == DN_BLOCKS * nb;
+            if (last) load_h();
+            stage_w(last ? m : mc, last ? it.chunk : chunk, last ? 0 : u + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            U.prepare(R, C, g, a.flag != 0 && row0 < a.rows, bad);
+            f32x16 c0 = zero16(), c1 = zero16();
+            const XRead x(sA[b][r], r, g);
+            uint4 xh = x(0, 0), xl = x(0, 512), nh, nl;
+            uint4 w0, r0, v0, q0;
+            U.template step<X0>(R, C, 0, w0, r0);
+#pragma unroll
+            for (int s = 0; s < 16; s++) {
+                if (s < 15) {
+                    nh = x(s + 1, 256 * ((s + 1) >> 3));
+                    nl = x(s + 1, 512 + 256 * ((s + 1) >> 3));
+                }
+                c0 = mfma32(xh, w0, c0);
+                c1 = mfma32(xl, w0, c1);
+                if (X0) c0 = mfma32(xh, r0, c0);
+                if (s < 15) U.template step<X0>(R, C, s + 1, v0, q0);
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, QT == Q4 ? 5 : 14, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                xh = nh;
+                xl = nl;
+                w0 = v0;
+                r0 = q0;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) c0[i] += c1[i];
+            uint4 sums = make_uint4(0, 0, 0, 0);
+            if (QT == Q4) sums = *reinterpret_cast<const uint4 *>(sS[b][r][g]);
+            U.add(R, sums, c0, t);
+            if (b == nb - 1) {
+                // rows past nr (and blocks past the end) fall outside the
+                // buffer's range: every lane issues all 16 stores, which the
+                // next unit's wait leaves in flight
+                const __amdgpu_buffer_rsrc_t ob =
+                    rsrc(a.eo + (size_t)p0 * a.rows, row0 < a.rows ? (uint32_t)(nr * a.rows * 4) : 0u);
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int n = 8 * (i >> 2) + 4 * g + (i & 3);
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ldexpf(t[i], sexp[n])), ob,
+                                                          4 * (uint32_t)(n * a.rows + row0 + r), 0, 0);
+                    t[i] = 0.f;
+                }
+                stores = true;
+            } else {
+                stores = false;
+            }
+        }
+        if (!more) break;
+        gg_bar();  // the tile's rows in LDS are read
     }
+    wait_vm<0>();  // (the loads past the end)
+    if (a.flag && __builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0)
+        __hip_atomic_fetch_or(a.err, BREAD_DEV_ERR_RANGE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // hidden[t] += sigmoid(gsh[t]) * shared(t), then += w_k * expert_k(t) for
@@ -818,21 +1137,32 @@ int max_tiles(const bread_moe_shape_t &s, int T)
     return P / MT + (P < s.n_experts ? P : s.n_experts) + (T + MT - 1) / MT;
 }
 
-// Tiles one XCD's list can hold: an eighth of the tiles plus one segment.
-int xcd_tiles(const bread_moe_shape_t &s, int T)
+// Workgroups for the items of at most `tiles` tiles of C chunks: what is
+// resident at once, whole XCDs.
+dim3 gg_grid(int tiles, int C, int resident)
 {
-    return (max_tiles(s, T) + NXCD - 1) / NXCD + SEG;
+    const int64_t items = (int64_t)tiles * C;
+    return dim3((unsigned)(((items < resident ? (int)items : resident) + NXCD - 1) / NXCD * NXCD));
 }
 
-int chunks_gu(const bread_moe_shape_t &s)
+void launch_gateup(const GgArgs &a, int tg, int tu, int tiles, int cus, hipStream_t st)
 {
-    const int Imax = s.expert_inter > s.shared_inter ? s.expert_inter : s.shared_inter;
-    return (Imax + GU_ROWS - 1) / GU_ROWS;
+    constexpr int Q4 = BREAD_QTYPE_Q4_K, Q6 = BREAD_QTYPE_Q6_K;
+    const dim3 grid = gg_grid(tiles, a.rows / GU_ROWS, 2 * cus), block(GG_THREADS);
+    if (tg == Q4 && tu == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q4>), grid, block, 0, st, a);
+    else if (tg == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q6>), grid, block, 0, st, a);
+    else if (tu == Q4) hipLaunchKernelGGL((k_gateup<Q6, Q4>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_gateup<Q6, Q6>), grid, block, 0, st, a);
 }
 
-int chunks_dn(const bread_moe_shape_t &s)
+// exact: Q6_K operands carry what fp16 rounds off
+void launch_down(const GgArgs &a, int td, bool exact, int tiles, int cus, hipStream_t st)
 {
-    return (s.hidden + DN_ROWS - 1) / DN_ROWS;
+    constexpr int Q4 = BREAD_QTYPE_Q4_K, Q6 = BREAD_QTYPE_Q6_K;
+    const dim3 grid = gg_grid(tiles, (a.rows + DN_ROWS - 1) / DN_ROWS, cus), block(DN_WAVES * WAVE);
+    if (td == Q4) hipLaunchKernelGGL((k_down_gg<Q4, true>), grid, block, 0, st, a);
+    else if (exact) hipLaunchKernelGGL((k_down_gg<Q6, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_down_gg<Q6, false>), grid, block, 0, st, a);
 }
 
 }  // namespace
@@ -848,16 +1178,17 @@ int bread_grouped_alloc(bread_moe_ctx_t *c)
     const size_t P = T * (K + 1);
     hipError_t e = hipSuccess;
     bread_grouped_ws &g = c->gws;
-    if (e == hipSuccess) e = hipMalloc(&g.xhi, T * H * 2);
-    if (e == hipSuccess) e = hipMalloc(&g.xlo, T * H * 2);
+    e = hipDeviceGetAttribute(&g.cus, hipDeviceAttributeMultiprocessorCount, c->device);
+    if (e == hipSuccess) e = hipMalloc(&g.xop, T * H * 4);
+    if (e == hipSuccess) e = hipMalloc(&g.xsum, T * (H / QK) * 32);
     if (e == hipSuccess) e = hipMalloc((void **)&g.xexp, T * sizeof(int));
     if (e == hipSuccess) e = hipMalloc((void **)&g.pair_tok, P * sizeof(int));
     if (e == hipSuccess) e = hipMalloc((void **)&g.pos_of, T * K * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&g.tiles, (size_t)max_tiles(s, c->max_tokens) * sizeof(MtTile));
-    if (e == hipSuccess) e = hipMalloc((void **)&g.n_tiles, sizeof(int));
-    const size_t xt = (size_t)xcd_tiles(s, c->max_tokens);
-    if (e == hipSuccess) e = hipMalloc((void **)&g.work, NXCD * xt * (chunks_gu(s) + chunks_dn(s)) * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc((void **)&g.n_work, 2 * NXCD * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc((void **)&g.n_tiles, 2 * sizeof(int));
+    const size_t Imax = (size_t)(s.expert_inter > s.shared_inter ? s.expert_inter : s.shared_inter);
+    if (e == hipSuccess && Imax <= MAX_INTER)
+        e = hipMalloc((void **)&g.h, (size_t)max_tiles(s, c->max_tokens) * MT * Imax * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void **)&g.eo, P * H * sizeof(float));
     return e == hipSuccess ? BREAD_OK : (e == hipErrorOutOfMemory ? BREAD_ERR_NOMEM : BREAD_ERR_HIP);
 }
@@ -865,15 +1196,14 @@ int bread_grouped_alloc(bread_moe_ctx_t *c)
 void bread_grouped_free(bread_moe_ctx_t *c)
 {
     bread_grouped_ws &g = c->gws;
-    (void)hipFree(g.xhi);
-    (void)hipFree(g.xlo);
+    (void)hipFree(g.xop);
+    (void)hipFree(g.xsum);
     (void)hipFree(g.xexp);
     (void)hipFree(g.pair_tok);
     (void)hipFree(g.pos_of);
     (void)hipFree(g.tiles);
     (void)hipFree(g.n_tiles);
-    (void)hipFree(g.work);
-    (void)hipFree(g.n_work);
+    (void)hipFree(g.h);
     (void)hipFree(g.eo);
     g = bread_grouped_ws{};
 }
@@ -881,7 +1211,7 @@ void bread_grouped_free(bread_moe_ctx_t *c)
 bool bread_grouped_supported(const bread_moe_shape_t &s, const bread_moe_layer_t *L)
 {
     if (s.expert_inter > MAX_INTER || s.shared_inter > MAX_INTER || !bread_standard_qtypes(L)) return false;
-    // Q6_K expert blocks must end 16-byte aligned (see the down operand order)
+    // 16-byte aligned Q6_K tensors, as the pinned path has always asked for
     const uintptr_t a16 = (uintptr_t)L->down_exps | (uintptr_t)L->down_shexp | L->down_expert_bytes;
     return (a16 & 15) == 0;
 }
@@ -905,44 +1235,65 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     }
     if ((E + WAVE - 1) / WAVE <= 4)
         hipLaunchKernelGGL(k_mt_topk_xprep<4>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x,
-                           (const uint16_t *)L->shexp_gate, H, (uint4 *)g.xhi, (uint4 *)g.xlo, g.xexp, c->gsh);
+                           (const uint16_t *)L->shexp_gate, H, (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, c->gsh);
     else
         hipLaunchKernelGGL(k_mt_topk_xprep<16>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x,
-                           (const uint16_t *)L->shexp_gate, H, (uint4 *)g.xhi, (uint4 *)g.xlo, g.xexp, c->gsh);
+                           (const uint16_t *)L->shexp_gate, H, (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, c->gsh);
     BREAD_HIP(hipGetLastError());
-    const int cgu = chunks_gu(s), cdn = chunks_dn(s);
-    const int slots_gu = xcd_tiles(s, T) * cgu, slots_dn = xcd_tiles(s, T) * cdn;
-    int *work_gu = g.work, *work_dn = g.work + (size_t)NXCD * slots_gu;
     hipLaunchKernelGGL(k_mt_bucket, dim3(1), dim3(1024), 0, st, c->idx, T, K, E, g.pair_tok, g.pos_of,
-                       (MtTile *)g.tiles, g.n_tiles, work_gu, work_dn, g.n_work, cgu, cdn, slots_gu, slots_dn);
+                       (MtTile *)g.tiles, g.n_tiles);
     BREAD_HIP(hipGetLastError());
-    MtArgs a;
-    a.L = *L;
+    const int tiles = max_tiles(s, T);
+    GgArgs a;
     a.err = &c->dsync->error.v;
-    a.H = H;
-    a.I = s.expert_inter;
-    a.Ish = s.shared_inter;
-    a.Imax = Imax;
-    a.E = E;
-    a.K = K;
-    a.T = T;
-    a.xhi = (const uint4 *)g.xhi;
-    a.xlo = (const uint4 *)g.xlo;
+    a.xop = (const uint4 *)g.xop;
+    a.xsum = (const uint4 *)g.xsum;
     a.xexp = g.xexp;
     a.pair_tok = g.pair_tok;
     a.tiles = (const MtTile *)g.tiles;
     a.n_tiles = g.n_tiles;
-    a.work_gu = work_gu;
-    a.work_dn = work_dn;
-    a.n_work = g.n_work;
-    a.slots_gu = slots_gu;
-    a.slots_dn = slots_dn;
-    a.h = c->h;
+    a.h = g.h;
     a.eo = g.eo;
-    hipLaunchKernelGGL(k_mt_gateup, dim3(NXCD * slots_gu), dim3(GU_WAVES * WAVE), 0, st, a);
+    a.E = E;
+    a.hstride = Imax;
+    const bool standard = bread_standard_qtypes(L);
+    a.flag = standard ? 1 : 0;
+    // one launch takes tiles of one geometry and type: the shared expert's
+    // ride along with the routed ones' where both agree
+    const bool one_gu = s.expert_inter == s.shared_inter && L->gate_type == L->gate_shexp_type &&
+                        L->up_type == L->up_shexp_type;
+    const bool one_dn = s.expert_inter == s.shared_inter && L->down_type == L->down_shexp_type;
+    a.w0 = (const uint8_t *)L->gate_exps;
+    a.w1 = (const uint8_t *)L->up_exps;
+    a.st0 = L->gate_expert_bytes;
+    a.st1 = L->up_expert_bytes;
+    a.sw0 = (const uint8_t *)L->gate_shexp;
+    a.sw1 = (const uint8_t *)L->up_shexp;
+    a.nsb = H / QK;
+    a.rows = s.expert_inter;
+    a.sel = one_gu ? 0 : 1;
+    launch_gateup(a, L->gate_type, L->up_type, tiles, g.cus, st);
     BREAD_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_mt_down, dim3(NXCD * slots_dn), dim3(DN_WAVES * WAVE), 0, st, a);
+    if (!one_gu) {
+        a.rows = s.shared_inter;
+        a.sel = 2;
+        launch_gateup(a, L->gate_shexp_type, L->up_shexp_type, tiles, g.cus, st);
+        BREAD_HIP(hipGetLastError());
+    }
+    a.w0 = a.w1 = (const uint8_t *)L->down_exps;
+    a.st0 = a.st1 = L->down_expert_bytes;
+    a.sw0 = a.sw1 = (const uint8_t *)L->down_shexp;
+    a.nsb = s.expert_inter / QK;
+    a.rows = H;
+    a.sel = one_dn ? 0 : 1;
+    launch_down(a, L->down_type, !standard, tiles, g.cus, st);
     BREAD_HIP(hipGetLastError());
+    if (!one_dn) {
+        a.nsb = s.shared_inter / QK;
+        a.sel = 2;
+        launch_down(a, L->down_shexp_type, !standard, tiles, g.cus, st);
+        BREAD_HIP(hipGetLastError());
+    }
     hipLaunchKernelGGL(k_mt_combine, dim3(T, (H / 4 + 255) / 256), dim3(256), 0, st, g.eo, g.pos_of, c->w, c->gsh,
                        hidden, H, K, T);
     BREAD_HIP(hipGetLastError());
