@@ -13,7 +13,7 @@
 // <= 63 * 15) or sc * (q - 32) (Q6_K, |.| <= 4096: exact up to 2048 and for
 // even values; the odd ones above are rounded to even in layers of the
 // reference GPU path's types and carried by a second operand in the others,
-// which ran in fp32 before).  Activations are two fp16 terms (hi + lo, 22
+// which keep fp32's precision), times a power of two.  Activations are two fp16 terms (hi + lo, 22
 // significant bits) after a power-of-two row scale into [2^13, 2^14) (exact,
 // undone on the fp32 result).  The superblock scale d, and for Q4_K the min
 // term dmin * sum_j m_j * (sum of x over sub-block j), are applied to the
@@ -383,7 +383,7 @@ __device__ __forceinline__ half2v pair(float a, float b)
     return half2v{(_Float16)a, (_Float16)b};
 }
 
-// Masks and magic numbers in registers: (v & mask) | magic is then one
+// Masks and magic numbers in registers: (v & mask) | w is then one
 // three-operand instruction (with literals, which that form does not take,
 // the compiler makes two).
 struct Consts {
@@ -415,60 +415,85 @@ __device__ __forceinline__ half2v pair_u8(uint32_t v)
 // the sums.  prepare() sets bad when the superblock is outside the range that
 // fp16 weights can hold (checked where `flag`): Q4_K |d| >= 64 or |dmin| >=
 // 1024, Q6_K |d sc| >= 2047, or NaN.
-template <int QT>
+template <int QT, bool X>
 struct Unit;
 
-template <>
-struct Unit<BREAD_QTYPE_Q4_K> {
-    half2v sc[2], ns[2];
+template <bool X>
+struct Unit<BREAD_QTYPE_Q4_K, X> {
+    half2v sc[2], ns[X ? 2 : 1];
 
-    // Scales of groups 0, 1 and 2, 3: a pair each; odd groups meet 16 q (the
-    // nibble left in place).  fma(1024 + q, sc, -1024 sc) = sc q exactly.
+    // Scales of groups 0, 1 and 2, 3: a pair each.  A masked nibble is the
+    // fp16 subnormal q 2^-24 (odd groups: 16 q 2^-24, left in place), and
+    //   q 2^-24 * sc 2^10 = sc q 2^-14,
+    // or with X fma(q 2^-24, sc 2^10, -8 sc 2^-14) = sc (q - 8) 2^-14, both
+    // exact.  The centred form halves the rounding of the sums and with it
+    // leaves the layer's error at that of the per-token kernels (5.7e-7
+    // against 5.8e-7 over 130 tokens; 6.0e-7 without); it costs gate/up 4 %.
     __device__ __forceinline__ void prepare(const Raw<BREAD_QTYPE_Q4_K> &R, const Consts &C, int g, bool flag, bool &bad)
     {
         const uint32_t s0 = R.hd.y, s2 = R.hd.w;
         if (flag) bad |= !(fabsf(h2f(R.hd.x)) < 64.f && fabsf(h2f(R.hd.x >> 16)) < 1024.f);
         const uint32_t sc4 = ((g ? s2 : s0) & C.sca) | ((s0 >> 2) & C.scb);
         const half2v p0 = pair_u8<0, 1>(sc4), p1 = pair_u8<2, 3>(sc4);
-        sc[0] = p0 * pair(1.f, 0.0625f);
-        sc[1] = p1 * pair(1.f, 0.0625f);
-        ns[0] = p0 * pair(-1024.f, -64.f);
-        ns[1] = p1 * pair(-1024.f, -64.f);
+        sc[0] = p0 * pair(1024.f, 64.f);
+        sc[1] = p1 * pair(1024.f, 64.f);
+        if constexpr (X) {
+            ns[0] = p0 * pair(-0x1p-11f, -0x1p-11f);
+            ns[1] = p1 * pair(-0x1p-11f, -0x1p-11f);
+        }
     }
 
-    // tot += d * c - dmin * sum_j m_j * (sum of x over sub-block j): m_0..7
-    // against the hi and lo sums
+    // tot += 2^14 d c - sum_j dmin m_j (sum of x over sub-block j), with X +
+    // sum_j 8 d sc_j of them: m_0..7 and sc_0..7 against the hi and lo sums.
+    // The last two are of one size and cancel, so they meet before the total.
     __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q4_K> &R, const uint4 &sums, const f32x16 &c,
                                         f32x16 &tot) const
     {
-        const uint32_t s1 = R.hd.z, s2 = R.hd.w;
-        const uint32_t ml = s1 & 0x3F3F3F3Fu, mh = ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u);
-        const uint4 mv = make_uint4(u_of(pair_u8<0, 1>(ml)), u_of(pair_u8<2, 3>(ml)), u_of(pair_u8<0, 1>(mh)),
-                                    u_of(pair_u8<2, 3>(mh)));
+        const uint32_t s0 = R.hd.y, s1 = R.hd.z, s2 = R.hd.w;
+        auto eight = [](uint32_t lo, uint32_t hi) __attribute__((always_inline)) {
+            return make_uint4(u_of(pair_u8<0, 1>(lo)), u_of(pair_u8<2, 3>(lo)), u_of(pair_u8<0, 1>(hi)),
+                              u_of(pair_u8<2, 3>(hi)));
+        };
+        const uint4 mv = eight(s1 & 0x3F3F3F3Fu, ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u));
         const f32x16 pm = mfma32(sums, mv, zero16());
-        const float d = h2f(R.hd.x), dm = -32.f * h2f(R.hd.x >> 16);
+        const float d = 16384.f * h2f(R.hd.x), dm = -32.f * h2f(R.hd.x >> 16);
+        if constexpr (X) {
+            const uint4 sv = eight(s0 & 0x3F3F3F3Fu, (s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u));
+            const f32x16 ps = mfma32(sums, sv, zero16());
+            const float d8 = 256.f * h2f(R.hd.x);
 #pragma unroll
-        for (int i = 0; i < 16; i++) tot[i] = fmaf(c[i], d, tot[i]);
+            for (int i = 0; i < 16; i++) tot[i] += fmaf(c[i], d, fmaf(pm[i], dm, ps[i] * d8));
+        } else {
 #pragma unroll
-        for (int i = 0; i < 16; i++) tot[i] = fmaf(pm[i], dm, tot[i]);
+            for (int i = 0; i < 16; i++) tot[i] = fmaf(c[i], d, tot[i]);
+#pragma unroll
+            for (int i = 0; i < 16; i++) tot[i] = fmaf(pm[i], dm, tot[i]);
+        }
     }
 
-    template <bool X>
     __device__ __forceinline__ void step(const Raw<BREAD_QTYPE_Q4_K> &R, const Consts &C, int s, uint4 &w, uint4 &) const
     {
         const int pp = s >> 3;
         const uint32_t v = comp(R.q[s >> 2], s & 3), v8 = v >> 8;
-        const half2v se = dup(sc[pp], 0), so = dup(sc[pp], 1), ne = dup(ns[pp], 0), no = dup(ns[pp], 1);
-        w = make_uint4(u_of(__builtin_elementwise_fma(h2_of((v & C.lo) | C.magic), se, ne)),
-                       u_of(__builtin_elementwise_fma(h2_of((v8 & C.lo) | C.magic), se, ne)),
-                       u_of(__builtin_elementwise_fma(h2_of((v & C.hi) | C.magic), so, no)),
-                       u_of(__builtin_elementwise_fma(h2_of((v8 & C.hi) | C.magic), so, no)));
+        const half2v se = dup(sc[pp], 0), so = dup(sc[pp], 1);
+        const half2v a0 = h2_of(v & C.lo), a1 = h2_of(v8 & C.lo), b0 = h2_of(v & C.hi), b1 = h2_of(v8 & C.hi);
+        if constexpr (X) {
+            const half2v ne = dup(ns[pp], 0), no = dup(ns[pp], 1);
+            w = make_uint4(u_of(__builtin_elementwise_fma(a0, se, ne)), u_of(__builtin_elementwise_fma(a1, se, ne)),
+                           u_of(__builtin_elementwise_fma(b0, so, no)), u_of(__builtin_elementwise_fma(b1, so, no)));
+        } else {
+            w = make_uint4(u_of(a0 * se), u_of(a1 * se), u_of(b0 * so), u_of(b1 * so));
+        }
     }
 };
 
-template <>
-struct Unit<BREAD_QTYPE_Q6_K> {
-    half2v sc[4];  // scales sc[8 g + 2 q], sc[8 g + 2 q + 1] of group q: elements 0..15 and 16..31
+template <bool X>
+struct Unit<BREAD_QTYPE_Q6_K, X> {
+    // scales sc[8 g + 2 q], sc[8 g + 2 q + 1] of group q, elements 0..15 and
+    // 16..31, times S: without X an element is the fp16 subnormal q 2^-24 and
+    // fma(q 2^-24, 2^8 sc, -32 sc 2^-16) rounds sc (q - 32) 2^-16 once
+    static constexpr float S = X ? 1.f : 256.f;
+    half2v sc[4], ns[X ? 1 : 4];
 
     __device__ __forceinline__ void prepare(const Raw<BREAD_QTYPE_Q6_K> &R, const Consts &, int, bool flag, bool &bad)
     {
@@ -483,18 +508,25 @@ struct Unit<BREAD_QTYPE_Q6_K> {
 #pragma unroll
             for (int q = 0; q < 8; q++) bad |= !(fabsf(d * (float)sc[q >> 1][q & 1]) < 2047.f);
         }
+        if constexpr (!X) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                ns[q] = sc[q] * pair(-0x1p-11f, -0x1p-11f);
+                sc[q] = sc[q] * pair(S, S);
+            }
+        }
     }
 
     __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q6_K> &R, const uint4 &, const f32x16 &c,
                                         f32x16 &tot) const
     {
-        const float d = h2f(R.d);
+        const float d = (X ? 1.f : 0x1p16f) * h2f(R.d);
 #pragma unroll
         for (int i = 0; i < 16; i++) tot[i] = fmaf(c[i], d, tot[i]);
     }
 
-    // w = fp16(sc (q - 32)); r (X): what that rounds off, 0 or +-1
-    template <bool X>
+    // w = fp16(sc (q - 32)), times 2^-16 without X; r (X): what that rounds
+    // off, 0 or +-1
     __device__ __forceinline__ void step(const Raw<BREAD_QTYPE_Q6_K> &R, const Consts &C, int s, uint4 &w, uint4 &r) const
     {
         const int pp = s >> 3, k = s & 7;
@@ -505,10 +537,16 @@ struct Unit<BREAD_QTYPE_Q6_K> {
             const int q = 2 * pp + (j >> 1), lsh = 4 * pp + 8 * (j & 1), hsh = 8 * (j & 1) + 2 * q - 4;
             const uint32_t l = R.l[(j >> 1) * 2 + (k >> 2)][k & 3] >> lsh;
             const uint32_t hb = hsh >= 0 ? h >> hsh : h << -hsh;
-            const half2v v = h2_of((hb & C.q2) | ((l & C.lo) | C.magic)) - pair(1056.f, 1056.f);  // q - 32, exact
-            const half2v se = dup(sc[q], k >> 2), p = v * se;
-            wv[j] = u_of(p);
-            rv[j] = X ? u_of(__builtin_elementwise_fma(v, se, -p)) : 0;
+            const half2v se = dup(sc[q], k >> 2);
+            if constexpr (X) {
+                const half2v v = h2_of((hb & C.q2) | ((l & C.lo) | C.magic)) - pair(1056.f, 1056.f);  // q - 32, exact
+                const half2v p = v * se;
+                wv[j] = u_of(p);
+                rv[j] = u_of(__builtin_elementwise_fma(v, se, -p));
+            } else {
+                wv[j] = u_of(__builtin_elementwise_fma(h2_of((hb & C.q2) | (l & C.lo)), se, dup(ns[q], k >> 2)));
+                rv[j] = 0;
+            }
         }
         w = make_uint4(wv[0], wv[1], wv[2], wv[3]);
         r = make_uint4(rv[0], rv[1], rv[2], rv[3]);
@@ -665,7 +703,8 @@ constexpr int W_CHUNKS = 32 * Q4K_BYTES / 16;  // 16-byte pieces of a matrix's s
 constexpr int W_LOADS = (W_CHUNKS + WAVE - 1) / WAVE;
 constexpr int W_BUF = W_LOADS * WAVE;  // the last load's idle lanes repeat the last piece
 
-template <int Q0, int Q1>
+// X: the exact operands of layers of other types than the reference GPU path's
+template <int Q0, int Q1, bool X>
 __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K;
@@ -753,16 +792,16 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
 
     const Consts C = consts(g);
     f32x16 t0 = zero16(), t1 = zero16(), c0, c1;
-    Unit<Q0> U0;
-    Unit<Q1> U1;
+    Unit<Q0, X> U0;
+    Unit<Q1, X> U1;
     bool bad = false;
     // steps 8 pp .. 8 pp + 7 of the superblock in R0, R1
     auto compute = [&](const uint4 (&sA)[MT][32], int pp) __attribute__((always_inline)) {
         const XRead x(sA[r], r, g);
         uint4 xh = x(0, 0), xl = x(0, 256), nh, nl;
         uint4 w0, w1, r0, r1, v0, v1, q0, q1;
-        U0.template step<X0>(R0, C, 8 * pp, w0, r0);
-        U1.template step<X1>(R1, C, 8 * pp, w1, r1);
+        U0.step(R0, C, 8 * pp, w0, r0);
+        U1.step(R1, C, 8 * pp, w1, r1);
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             if (s < 7) {
@@ -776,8 +815,8 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
             if (X0) c0 = mfma32(xh, r0, c0);
             if (X1) c1 = mfma32(xh, r1, c1);
             if (s < 7) {
-                U0.template step<X0>(R0, C, 8 * pp + s + 1, v0, q0);
-                U1.template step<X1>(R1, C, 8 * pp + s + 1, v1, q1);
+                U0.step(R0, C, 8 * pp + s + 1, v0, q0);
+                U1.step(R1, C, 8 * pp + s + 1, v1, q1);
             }
             // an MFMA, then VALU: the next step's operands are made under
             // this one's products
@@ -875,11 +914,12 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
 // buffer for the next one (loads of 16 bytes of a row a lane, 2-byte aligned,
 // took the address unit a cycle a lane).  The next item's SwiGLU rows and
 // first unit are requested while the last units run.
-// Measured as above, a lane a weight row / this: 64 tokens 23 / 23 us, 512
-// tokens 98 / 95 us, 2048 tokens 221 / 230 us (exact integer operands, a third
-// of the error).  A unit of 32 MFMA takes 3,500 cycles in its steps (VALU: a
-// Q6_K operand is some 20 instructions), 2,000 in its loads and its move to
-// registers.
+// Measured as above, a lane a weight row / this: 64 tokens 23 / 21 us, 512
+// tokens 98 / 91 us, 2048 tokens 221 / 208 us (a third of the error).  A unit
+// of 32 MFMA is bound by the VALU in its steps (a Q6_K operand pair is a mask,
+// a merge and a multiply-add on subnormals besides its shifts; with the
+// integers biased by 1024 and two more instructions a pair 23 / 100 / 230 us),
+// and takes 2,000 cycles in its loads and its move to registers.
 // ---------------------------------------------------------------------------
 
 // 16-byte pieces a row of a unit takes in the wave's buffer: a Q4_K superblock
@@ -919,6 +959,7 @@ __device__ __forceinline__ void take_unit(Raw<BREAD_QTYPE_Q6_K> &R, const uint4 
     R.d = p[52] >> (8 * sh);
 }
 
+// X as in k_gateup
 template <int QT, bool X>
 __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
 {
@@ -1016,7 +1057,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
     const Consts C = consts(g);
     f32x16 t = zero16();
     Raw<QT> R;
-    Unit<QT> U;
+    Unit<QT, X> U;
     bool bad = false;
     const uint8_t *m = matrix();
     bool stores = false;  // the last unit stored
@@ -1046,7 +1087,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
             const XRead x(sA[b][r], r, g);
             uint4 xh = x(0, 0), xl = x(0, 512), nh, nl;
             uint4 w0, r0, v0, q0;
-            U.template step<X0>(R, C, 0, w0, r0);
+            U.step(R, C, 0, w0, r0);
 #pragma unroll
             for (int s = 0; s < 16; s++) {
                 if (s < 15) {
@@ -1056,7 +1097,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
                 c0 = mfma32(xh, w0, c0);
                 c1 = mfma32(xl, w0, c1);
                 if (X0) c0 = mfma32(xh, r0, c0);
-                if (s < 15) U.template step<X0>(R, C, s + 1, v0, q0);
+                if (s < 15) U.step(R, C, s + 1, v0, q0);
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
                     __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
@@ -1145,24 +1186,25 @@ dim3 gg_grid(int tiles, int C, int resident)
     return dim3((unsigned)(((items < resident ? (int)items : resident) + NXCD - 1) / NXCD * NXCD));
 }
 
-void launch_gateup(const GgArgs &a, int tg, int tu, int tiles, int cus, hipStream_t st)
+// exact: layers of other types than the reference GPU path's (Unit)
+void launch_gateup(const GgArgs &a, int tg, int tu, bool exact, int tiles, int cus, hipStream_t st)
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K, Q6 = BREAD_QTYPE_Q6_K;
     const dim3 grid = gg_grid(tiles, a.rows / GU_ROWS, 2 * cus), block(GG_THREADS);
-    if (tg == Q4 && tu == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q4>), grid, block, 0, st, a);
-    else if (tg == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q6>), grid, block, 0, st, a);
-    else if (tu == Q4) hipLaunchKernelGGL((k_gateup<Q6, Q4>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_gateup<Q6, Q6>), grid, block, 0, st, a);
+    if (!exact) hipLaunchKernelGGL((k_gateup<Q4, Q4, false>), grid, block, 0, st, a);
+    else if (tg == Q4 && tu == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q4, true>), grid, block, 0, st, a);
+    else if (tg == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q6, true>), grid, block, 0, st, a);
+    else if (tu == Q4) hipLaunchKernelGGL((k_gateup<Q6, Q4, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_gateup<Q6, Q6, true>), grid, block, 0, st, a);
 }
 
-// exact: Q6_K operands carry what fp16 rounds off
 void launch_down(const GgArgs &a, int td, bool exact, int tiles, int cus, hipStream_t st)
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K, Q6 = BREAD_QTYPE_Q6_K;
     const dim3 grid = gg_grid(tiles, (a.rows + DN_ROWS - 1) / DN_ROWS, cus), block(DN_WAVES * WAVE);
-    if (td == Q4) hipLaunchKernelGGL((k_down_gg<Q4, true>), grid, block, 0, st, a);
-    else if (exact) hipLaunchKernelGGL((k_down_gg<Q6, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_down_gg<Q6, false>), grid, block, 0, st, a);
+    if (!exact) hipLaunchKernelGGL((k_down_gg<Q6, false>), grid, block, 0, st, a);
+    else if (td == Q4) hipLaunchKernelGGL((k_down_gg<Q4, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_down_gg<Q6, true>), grid, block, 0, st, a);
 }
 
 }  // namespace
@@ -1211,7 +1253,7 @@ void bread_grouped_free(bread_moe_ctx_t *c)
 bool bread_grouped_supported(const bread_moe_shape_t &s, const bread_moe_layer_t *L)
 {
     if (s.expert_inter > MAX_INTER || s.shared_inter > MAX_INTER || !bread_standard_qtypes(L)) return false;
-    // 16-byte aligned Q6_K tensors, as the pinned path has always asked for
+    // 16-byte aligned down weights, which the down kernel's loads ask for
     const uintptr_t a16 = (uintptr_t)L->down_exps | (uintptr_t)L->down_shexp | L->down_expert_bytes;
     return (a16 & 15) == 0;
 }
@@ -1227,18 +1269,24 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     bread_grouped_ws &g = c->gws;
     bread_clear_stale_error();
     // router logits in the reference's order (route.hip), then per token the
-    // exact softmax / top-k with the activation preparation
+    // exact softmax / top-k with the activation preparation.  The shared-gate
+    // score: summed in parallel there, or, for layers that keep the precision
+    // of the per-token kernels, in the reference's order too
+    const bool standard = bread_standard_qtypes(L);
+    const uint16_t *shg = (const uint16_t *)L->shexp_gate;
+    float *gsh = standard ? c->gsh : nullptr;
     {
-        const int rc = bread_launch_route_logits((const float *)L->router, nullptr, x, c->logits, nullptr, H, E, T,
-                                                 false, st);
+        const int rc = bread_launch_route_logits((const float *)L->router, standard ? nullptr : shg, x, c->logits,
+                                                 standard ? nullptr : c->gsh, H, E, T, !standard, st);
         if (rc) return rc;
     }
+    if (!standard) shg = nullptr;
     if ((E + WAVE - 1) / WAVE <= 4)
-        hipLaunchKernelGGL(k_mt_topk_xprep<4>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x,
-                           (const uint16_t *)L->shexp_gate, H, (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, c->gsh);
+        hipLaunchKernelGGL(k_mt_topk_xprep<4>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x, shg, H,
+                           (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, gsh);
     else
-        hipLaunchKernelGGL(k_mt_topk_xprep<16>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x,
-                           (const uint16_t *)L->shexp_gate, H, (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, c->gsh);
+        hipLaunchKernelGGL(k_mt_topk_xprep<16>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x, shg, H,
+                           (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, gsh);
     BREAD_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_mt_bucket, dim3(1), dim3(1024), 0, st, c->idx, T, K, E, g.pair_tok, g.pos_of,
                        (MtTile *)g.tiles, g.n_tiles);
@@ -1256,7 +1304,6 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     a.eo = g.eo;
     a.E = E;
     a.hstride = Imax;
-    const bool standard = bread_standard_qtypes(L);
     a.flag = standard ? 1 : 0;
     // one launch takes tiles of one geometry and type: the shared expert's
     // ride along with the routed ones' where both agree
@@ -1272,12 +1319,12 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     a.nsb = H / QK;
     a.rows = s.expert_inter;
     a.sel = one_gu ? 0 : 1;
-    launch_gateup(a, L->gate_type, L->up_type, tiles, g.cus, st);
+    launch_gateup(a, L->gate_type, L->up_type, !standard, tiles, g.cus, st);
     BREAD_HIP(hipGetLastError());
     if (!one_gu) {
         a.rows = s.shared_inter;
         a.sel = 2;
-        launch_gateup(a, L->gate_shexp_type, L->up_shexp_type, tiles, g.cus, st);
+        launch_gateup(a, L->gate_shexp_type, L->up_shexp_type, !standard, tiles, g.cus, st);
         BREAD_HIP(hipGetLastError());
     }
     a.w0 = a.w1 = (const uint8_t *)L->down_exps;
