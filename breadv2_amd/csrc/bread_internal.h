@@ -168,9 +168,10 @@ __host__ __device__ inline uint64_t bread_expert_row_bytes(int t, int cols)
     return (uint64_t)(cols / 256) * (t == BREAD_QTYPE_Q4_K ? 144u : 210u);
 }
 
-// The layout the specialised kernels (decode, small-batch, grouped) take:
-// Q4_K gate and up, Q6_K down, for the routed experts and the shared one.
-// Other mixes run on the per-token kernels.
+// The layout the decode and small-batch kernels take: Q4_K gate and up, Q6_K
+// down, for the routed experts and the shared one.  Other mixes run on the
+// per-token kernels or, for more tokens, the grouped ones (moe.hip,
+// grouped_takes_mix).
 inline bool bread_standard_qtypes(const bread_moe_layer_t *L)
 {
     return L->gate_type == BREAD_QTYPE_Q4_K && L->up_type == BREAD_QTYPE_Q4_K && L->down_type == BREAD_QTYPE_Q6_K &&

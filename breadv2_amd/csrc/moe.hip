@@ -544,6 +544,25 @@ extern "C" int bread_stack_loop_tokens(void)
     return 4;
 }
 
+// Whether a layer of another mix of Q4_K and Q6_K than the decode kernel's
+// goes to the grouped path rather than to the per-token kernels, which stream
+// an expert's rows once for every token that chose it.  us a layer on MI355X
+// (hidden 2048, intermediate 512, 256 experts, top 8, uniform routing),
+// per-token / grouped:
+//   tokens               2          3         4          6          8         27         130
+//   all Q4_K           61 / 68   78 / 70   88 / 71   120 / 75   151 / 79   421 / 146  1765 / 206
+//   all Q6_K           61 / 102  79 / 110  95 / 112  131 / 116  165 / 120  451 / 236  1886 / 360
+//   Q6_K shared down   60 / 85   77 / 87   87 / 89   119 / 93   152 / 99   423 / 163  1774 / 225
+// (Q6_K gate and up weights are gathered a row a lane; a shared expert of
+// another type takes launches of its own).
+static bool grouped_takes_mix(const bread_moe_layer_t *L, int T, const float *hidden)
+{
+    const int Q4 = BREAD_QTYPE_Q4_K;
+    const bool all_q4 = L->gate_type == Q4 && L->up_type == Q4 && L->down_type == Q4 && L->gate_shexp_type == Q4 &&
+                        L->up_shexp_type == Q4 && L->down_shexp_type == Q4;
+    return T >= (all_q4 ? 3 : 6) && ((uintptr_t)hidden & 15) == 0;
+}
+
 extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L, const float *x, float *hidden,
                                  int T, int32_t *idx, float *w, float *gsh, bread_stream_t stream)
 {
@@ -555,7 +574,7 @@ extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L,
     c->last_stream = st;
     if (c->path == BREAD_PATH_DECODE || c->path == BREAD_PATH_GROUPED || c->path == BREAD_PATH_SMALL)
         BREAD_REQUIRE(bread_standard_qtypes(L), BREAD_ERR_QTYPE,
-                      "the decode, small-batch and grouped kernels take Q4_K gate/up and Q6_K down "
+                      "pinned, the decode, small-batch and grouped paths take Q4_K gate/up and Q6_K down "
                       "(BREAD_PATH_PER_TOKEN and BREAD_PATH_AUTO take any mix of Q4_K and Q6_K)");
     switch (c->path) {
     case BREAD_PATH_DECODE:
@@ -577,7 +596,8 @@ extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L,
     default:
         rc = (T == 1) ? bread_launch_moe_decode(c, L, x, hidden, st) : BREAD_ERR_SHAPE;
         if (rc == BREAD_ERR_SHAPE && T <= bread_small_auto_tokens()) rc = bread_launch_moe_small(c, L, x, hidden, T, st);
-        if (rc == BREAD_ERR_SHAPE) rc = bread_launch_moe_grouped(c, L, x, hidden, T, st);
+        if (rc == BREAD_ERR_SHAPE && (bread_standard_qtypes(L) || grouped_takes_mix(L, T, hidden)))
+            rc = bread_launch_moe_grouped(c, L, x, hidden, T, st);
         if (rc == BREAD_ERR_SHAPE) rc = bread_launch_moe_multi(c, L, x, hidden, T, st);
     }
     if (rc) return rc;

@@ -124,9 +124,10 @@ void bread_moe_shape_default(bread_moe_shape_t *shape);
  * given per tensor as the reference records them (loader.c:191-193) and as its
  * fp32 path dispatches on them (one_layer.cu:1465-1468, layer_ops.cu:169-189).
  * Q4_K tensors and expert strides are 16-byte aligned, Q6_K ones 4-byte
- * aligned.  The decode, small-batch and grouped kernels take the mix the
- * reference GPU path hardcodes (gate/up Q4_K, down Q6_K, routed and shared,
- * one_layer.cu:1966-1977); any other mix runs on the per-token kernels.
+ * aligned.  The decode and small-batch kernels take the mix the reference GPU
+ * path hardcodes (gate/up Q4_K, down Q6_K, routed and shared,
+ * one_layer.cu:1966-1977); any other mix runs on the per-token kernels or, for
+ * more tokens, the grouped ones.
  * router F32 [E][H]; shexp_gate F16 [H] or NULL (NULL means a zero logit,
  * sigmoid 0.5, as when the reference finds no tensor, one_layer.cu:974-976). */
 typedef struct {
@@ -268,8 +269,11 @@ int bread_route_layer_f16(bread_moe_ctx_t *ctx, const bread_moe_layer_t *layer, 
  * it, fp32; H <= 2048, intermediate sizes 256 or 512); larger batches run the
  * grouped path (tokens bucketed by expert, expert GEMMs on the matrix cores
  * with fp16 operands and fp32 accumulation; intermediate sizes <= 512 and
- * 16-byte aligned Q6_K down weights); other shapes and weight-type mixes run
- * the per-token path.  A pinned path that cannot take the layer's weight
+ * 16-byte aligned Q6_K down weights); other shapes run the per-token path.
+ * Other weight-type mixes run the grouped path from a few tokens on (3 where
+ * every tensor is Q4_K, 6 otherwise; shapes and alignment as above, d_hidden
+ * 16-byte aligned) with operands that keep fp32's precision, and the
+ * per-token path else.  A pinned path that does not take the layer's weight
  * types returns BREAD_ERR_QTYPE. */
 int bread_moe_forward(bread_moe_ctx_t *ctx, const bread_moe_layer_t *layer,
                       const float *d_x_normed, float *d_hidden, int n_tokens,
