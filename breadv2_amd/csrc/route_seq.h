@@ -10,22 +10,34 @@
 // chain, so the kernel's time is a lane's H columns of (product, add) at the
 // issue rate of one wave; everything else is kept off that path.
 //   - Activations travel HBM/L2 -> LDS by gfx950 direct-to-LDS loads in
-//     chunks of 128 columns, RS_NB - 1 chunks in flight.  A token's chunk
-//     row is 32 16-byte units stored XOR-swizzled (unit u at u ^ (token %
-//     16)), so a wave's loads write contiguous LDS and the 16-byte reads of
-//     16 consecutive lanes fall in distinct banks.  Rows past the last token
-//     repeat the wave's router chunk (no lane reads them): activation rows
-//     that do not exist would otherwise all read one line.
-//   - Router rows are the same for every lane: a row's chunk sits in two
-//     registers in each 16-lane row of the wave (lane j: columns 4j .. 4j+3
-//     of each 64-column half) and each product takes its weight by DPP
-//     row_newbcast inside the v_mul, with no LDS traffic and no extra
-//     instruction.  The fp16 shared gate travels raw (every wave loads it)
-//     and the gate wave widens it when its chunk is used.
-//   - With direct-to-LDS loads in the kernel the compiler waits for every
-//     LDS read before the first use of any; the block reads are issued
-//     right after that wait, a block ahead, so it covers only reads that
-//     had a block's time to land.
+//     chunks of 64 columns through a ring of four buffers, up to four chunks
+//     ahead.  A buffer is a variable of its own and the loop is unrolled over
+//     the ring: a read of a variable that a direct-to-LDS load may still
+//     write waits for that load, and with one variable for all buffers every
+//     read waited for the loads that had just gone out.  A token's chunk row
+//     is 16 16-byte units stored XOR-swizzled (unit u at u ^ (token % 16)),
+//     so a wave's loads write contiguous LDS and the 16-byte reads of 16
+//     consecutive lanes fall in distinct banks.  Rows past the last token
+//     repeat earlier ones in turn (no lane's result is stored).
+//   - Router rows are the same for every lane: a row's chunk sits in one
+//     register quad in each 16-lane row of the wave (lane j: columns 4j ..
+//     4j+3) and each product takes its weight by DPP row_newbcast inside the
+//     v_mul, with no LDS traffic and no extra instruction.
+//   - The chain never drains: LDS reads run two blocks of 16 columns ahead
+//     and products one, across chunk borders too; a chunk's barrier stands
+//     two blocks before its end, where its last reads have returned (so its
+//     buffer is free) and the next chunk's first ones go out.
+// Loads past the last chunk repeat it into buffers that nothing reads, so
+// the counts that the waits rely on hold to the end.
+//
+// Bound: one wave a SIMD issues an instruction every 2.4 ns, so 2048 columns
+// of a product and an add take 10 us; where waves share a SIMD the DPP product
+// takes 2.2 ns and the add 1.1.  Measured on MI355X at 256 experts, hidden
+// 2048, against two 128-column buffers in one variable, a barrier and a drained
+// pipeline at each chunk: 64 tokens 19.6 -> 16.3 us, 512 tokens 31.5 -> 26.7
+// us, 2048 tokens 95 us both.  Weights by scalar loads two blocks ahead (a
+// plain product takes half a DPP one's issue): 57 / 59 / 115 us, the loads'
+// latency.
 #pragma once
 
 #include "bread_device.h"
@@ -34,27 +46,17 @@ namespace route_seq {
 
 constexpr int RS_WAVES = 4;              // waves per workgroup
 constexpr int RS_TT = WAVE;              // tokens per tile, one a lane
-constexpr int RS_CJ = 128;               // columns per staged chunk
-constexpr int RS_NB = 2;                 // chunk buffers (2 or 4): loads run RS_NB - 1 chunks ahead
+constexpr int RS_CJ = 64;                // columns per staged chunk
+constexpr int RS_NB = 4;                 // chunk buffers, and the chunks a loop pass covers
 constexpr int RS_BLK = 16;               // columns per block of the pipelined inner loop
-constexpr int RS_XI = RS_TT / 2 / RS_WAVES;  // activation loads a wave issues per chunk (8)
+constexpr int RS_XI = RS_TT / 4 / RS_WAVES;  // activation loads a wave issues per chunk
 
-static_assert(RS_CJ == 128 && RS_TT % (2 * RS_WAVES) == 0, "a wave instruction stages two 512-byte rows");
+static_assert(RS_CJ == 64 && RS_XI == 4, "a wave instruction stages four 256-byte rows");
 
-struct RsSmem {
-    float x[RS_NB][RS_TT][RS_CJ];  // the tile's activations by chunk, units swizzled
-};
+typedef float RsBuf[RS_TT][RS_CJ];  // a chunk of the tile's activations, units swizzled
 
 // Native 4-float vectors (HIP's float4 struct is copied through memory).
 typedef float rs_f4 __attribute__((ext_vector_type(4)));
-
-// Direct-to-LDS load (gfx950 global_load_lds_dwordx4): lane i of the wave
-// writes its 16 bytes at lds_wave_base + 16 i; the base must be
-// wave-uniform.  The data is in LDS once the issuing wave's vmcnt drains.
-__device__ __forceinline__ void lds_load16(const void *src, void *lds_wave_base)
-{
-    __builtin_amdgcn_global_load_lds(src, lds_wave_base, 16, 0, 0);
-}
 
 // s_waitcnt on the vector memory counter only (gfx9 encoding: vmcnt in
 // bits 3:0 and 15:14, expcnt and lgkmcnt left at their maxima).
@@ -68,11 +70,10 @@ __device__ __forceinline__ void wait_vm()
 // Keeps the vector memory operations issued before it ahead of those issued
 // after it.  The partial vmcnt waits of rs_run count on that order (gfx9
 // completes a wave's vector memory operations in issue order), and nothing
-// else pins it: the weight and gate loads read __restrict__ read-only
-// arguments, so the optimiser could hoist them above the direct-to-LDS
-// batch, and a wait meant for the batch would then leave part of it in
-// flight across the barrier.  The empty asm with a memory clobber stops the
-// optimiser, the scheduling barrier the machine scheduler.
+// else pins it: were a chunk's weights issued ahead of its activations, a
+// wait meant for those would leave part of them in flight across the barrier.
+// The empty asm with a memory clobber stops the optimiser, the scheduling
+// barrier the machine scheduler.
 __device__ __forceinline__ void issue_order()
 {
     asm volatile("" ::: "memory");
@@ -88,56 +89,6 @@ __device__ __forceinline__ void bar()
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-// Chunk c into buffer b: RS_XI direct-to-LDS loads a wave, two activation
-// rows an instruction (lanes 0-31 row 2i, 32-63 row 2i+1; lane l writes unit
-// l % 32 from unit (l % 32) ^ (row % 16) of the token's chunk).  Rows past
-// T load the same units of fb instead.
-__device__ __forceinline__ void rs_stage(RsSmem &S, int b, const float *__restrict__ x, const float *fb, int t0,
-                                         int T, int H, int c, int wv, int lane)
-{
-    const int half = lane >> 5, u = lane & 31;
-#pragma unroll
-    for (int i = 0; i < RS_XI; i++) {
-        const int row = 2 * (wv + RS_WAVES * i) + half;
-        const float *base = t0 + row < T ? x + (size_t)(t0 + row) * H : fb;
-        lds_load16(base + c * RS_CJ + 4 * (u ^ (row & 15)), &S.x[b][row - half][0]);
-    }
-}
-
-// The weights of chunk c for the wave's NE rows (w0 and the rows after it)
-// and the raw fp16 gate's (four halves a lane; g is a valid stand-in when
-// the wave has no gate).  Both are loaded by every wave: a choice between
-// loads would make the compiler wait for them where it merges the two.
-template <int NE>
-__device__ __forceinline__ void rs_load_w(rs_f4 (&w)[NE][2], uint2 (&gw)[2], const float *w0,
-                                          const uint16_t *__restrict__ g, int H, int c, int lane)
-{
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int col = c * RS_CJ + 64 * h + 4 * (lane & 15);
-        gw[h] = *reinterpret_cast<const uint2 *>(g + col);
-#pragma unroll
-        for (int n = 0; n < NE; n++) w[n][h] = *reinterpret_cast<const rs_f4 *>(w0 + (size_t)n * H + col);
-    }
-}
-
-// The weights chunk_dot reads: the rows', or for the gate wave the gate's
-// widened in place of row 0.
-template <int NE>
-__device__ __forceinline__ void rs_take(rs_f4 (&wc)[NE][2], const rs_f4 (&w)[NE][2], const uint2 (&gw)[2], bool gate)
-{
-#pragma unroll
-    for (int n = 0; n < NE; n++) {
-        wc[n][0] = w[n][0];
-        wc[n][1] = w[n][1];
-    }
-    if (gate) {
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-            wc[0][h] = rs_f4{h2f(gw[h].x), h2f(gw[h].x >> 16), h2f(gw[h].y), h2f(gw[h].y >> 16)};
-    }
 }
 
 // Lane n of each 16-lane row of v, to the whole row (DPP row_newbcast; the
@@ -171,18 +122,24 @@ __device__ __forceinline__ float row_bcast(float v, int n)
     }
 }
 
-// Router weight of chunk column col (0..127).
-__device__ __forceinline__ float rs_weight(const rs_f4 (&w)[2], int col)
+// Four halves widened.
+__device__ __forceinline__ rs_f4 widen(uint2 g)
 {
-    return row_bcast(w[col >> 6][col & 3], (col & 63) >> 2);
+    return rs_f4{h2f(g.x), h2f(g.x >> 16), h2f(g.y), h2f(g.y >> 16)};
 }
 
-// The lane's activations of one 16-column block from its swizzled LDS row.
-__device__ __forceinline__ void rs_load_x(const float *xrow, int sw, int blk, float (&xv)[RS_BLK])
+// Column col (0..63) of a row's chunk.
+__device__ __forceinline__ float rs_weight(const rs_f4 &w, int col)
+{
+    return row_bcast(w[col & 3], col >> 2);
+}
+
+// The lane's activations of one 16-column block of a chunk.
+__device__ __forceinline__ void rs_load_x(const RsBuf &buf, int lane, int blk, float (&xv)[RS_BLK])
 {
 #pragma unroll
     for (int q = 0; q < RS_BLK / 4; q++) {
-        const rs_f4 x4 = *reinterpret_cast<const rs_f4 *>(xrow + 4 * ((blk * (RS_BLK / 4) + q) ^ sw));
+        const rs_f4 x4 = *reinterpret_cast<const rs_f4 *>(&buf[lane][4 * ((blk * (RS_BLK / 4) + q) ^ (lane & 15))]);
         xv[4 * q] = x4[0];
         xv[4 * q + 1] = x4[1];
         xv[4 * q + 2] = x4[2];
@@ -190,132 +147,165 @@ __device__ __forceinline__ void rs_load_x(const float *xrow, int sw, int blk, fl
     }
 }
 
-// acc[n] += w_n[j] * x[j] for the chunk's 128 columns in order, each product
-// rounded before its add.  The adds of a lane are one dependent chain, so
-// the schedule is pinned: the adds of block b alternate with the
-// independent products of block b+1, and the LDS reads of block b+2 go out
-// right after the first of those products (the compiler's wait for all LDS
-// reads sits before it).  Every lane of the wave runs it: the weights come
-// from other lanes by DPP.
-template <int NE>
-__device__ __forceinline__ void chunk_dot(const float *xrow, int sw, const rs_f4 (&w)[NE][2], float (&acc)[NE])
+// The sums of one wave: acc[n] += w_n[j] x[j] for j = 0 .. H - 1 in order,
+// each product rounded before its add, w_n the rows from w0, or (GATE, NE 1)
+// the fp16 row g.  x: the tile's first row, nt its tokens.  Every wave of the
+// workgroup runs it (all of them stage), every lane too (the weights come
+// from other lanes by DPP).  H % 256 == 0.
+template <int NE, bool GATE>
+__device__ __forceinline__ void rs_run(RsBuf &b0, RsBuf &b1, RsBuf &b2, RsBuf &b3, const float *__restrict__ x, int nt,
+                                       const float *__restrict__ w0, const uint16_t *__restrict__ g, int H,
+                                       float (&acc)[NE])
 {
 #pragma clang fp contract(off)
-    constexpr int NBK = RS_CJ / RS_BLK;
-    float x1[RS_BLK], x2[RS_BLK];
-    float p[NE][RS_BLK], pn[NE][RS_BLK];
-    rs_load_x(xrow, sw, 0, x1);
+    static_assert(!GATE || NE == 1, "one gate row");
+    constexpr int BPC = RS_CJ / RS_BLK;       // blocks a chunk
+    constexpr int PER = RS_XI + NE;           // loads of a chunk: activations, then weights
+    const int lane = lane_id(), wv = wave_id();
+    const int nc = H / RS_CJ;
+    // lane l of a load writes unit l % 16 of row l / 16 from unit (l % 16) ^
+    // (row % 16) of the token's chunk
+    const __amdgpu_buffer_rsrc_t xb = rsrc(x, 4u * (uint32_t)(nt * H));
+    uint32_t xo[RS_XI];
+#pragma unroll
+    for (int i = 0; i < RS_XI; i++) {
+        const int row = 4 * (wv + RS_WAVES * i) + (lane >> 4);
+        xo[i] = 4u * (uint32_t)((row % nt) * H + 4 * ((lane & 15) ^ (row & 15)));
+    }
+    auto stage = [&](RsBuf &b, int c, int i) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, &b[4 * (wv + RS_WAVES * i)][0], 16, xo[i],
+                                                 4 * RS_CJ * min(c, nc - 1), 0, 0);
+    };
+    // (buffer loads: plain ones from read-only arguments would not stay where
+    // they are issued)
+    const __amdgpu_buffer_rsrc_t wb = GATE ? rsrc(g, 2u * (uint32_t)H) : rsrc(w0, 4u * (uint32_t)(NE * H));
+    rs_f4 wr[RS_NB][NE];
+    uint2 gr[RS_NB];
+    const uint32_t wo = (GATE ? 8 : 16) * (lane & 15);
+    auto load_w = [&](int k, int c) __attribute__((always_inline)) {
+        const int col = min(c, nc - 1) * RS_CJ;
+        if constexpr (GATE) {
+            gr[k] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(wb, wo, 2 * col, 0));
+        } else {
+#pragma unroll
+            for (int n = 0; n < NE; n++)
+                wr[k][n] = __builtin_bit_cast(rs_f4, __builtin_amdgcn_raw_buffer_load_b128(wb, wo, 4 * (n * H + col), 0));
+        }
+    };
+    auto weight = [&](int k, int n, int col) __attribute__((always_inline)) {
+        if constexpr (GATE) return rs_weight(widen(gr[k]), col);
+        else return rs_weight(wr[k][n], col);
+    };
+    auto read = [&](int k, int blk, float (&xv)[RS_BLK]) __attribute__((always_inline)) {
+        if (k == 0) rs_load_x(b0, lane, blk, xv);
+        else if (k == 1) rs_load_x(b1, lane, blk, xv);
+        else if (k == 2) rs_load_x(b2, lane, blk, xv);
+        else rs_load_x(b3, lane, blk, xv);
+    };
+    auto stage_k = [&](int k, int c, int i) __attribute__((always_inline)) {
+        if (k == 0) stage(b0, c, i);
+        else if (k == 1) stage(b1, c, i);
+        else if (k == 2) stage(b2, c, i);
+        else stage(b3, c, i);
+    };
+    float x1[RS_BLK], x2[RS_BLK], p[NE][RS_BLK], pn[NE][RS_BLK];
+#pragma unroll
+    for (int k = 0; k < RS_NB; k++) {
+#pragma unroll
+        for (int i = 0; i < RS_XI; i++) stage_k(k, k, i);
+        issue_order();
+        load_w(k, k);
+        issue_order();
+    }
+    wait_vm<NE + (RS_NB - 1) * PER>();
+    bar();
+    read(0, 0, x1);
 #pragma unroll
     for (int j = 0; j < RS_BLK; j++)
 #pragma unroll
-        for (int n = 0; n < NE; n++) p[n][j] = rs_weight(w[n], j) * x1[j];
-    rs_load_x(xrow, sw, 1, x1);
+        for (int n = 0; n < NE; n++) p[n][j] = weight(0, n, j) * x1[j];
+    read(0, 1, x1);
+    for (int c = 0; c < nc; c += RS_NB) {
 #pragma unroll
-    for (int blk = 0; blk < NBK; blk++) {
+        for (int k = 0; k < RS_NB; k++) {
 #pragma unroll
-        for (int j = 0; j < RS_BLK; j++) {
+            for (int bl = 0; bl < BPC; bl++) {
+                const int kn = (bl + 1) / BPC ? (k + 1) % RS_NB : k, bn = (bl + 1) % BPC;  // the next block
+                const int kr = (bl + 2) / BPC ? (k + 1) % RS_NB : k, br = (bl + 2) % BPC;  // the one after it
 #pragma unroll
-            for (int n = 0; n < NE; n++) acc[n] = acc[n] + p[n][j];
-            if (blk + 1 < NBK) {
+                for (int j = 0; j < RS_BLK; j++) {
 #pragma unroll
-                for (int n = 0; n < NE; n++) pn[n][j] = rs_weight(w[n], (blk + 1) * RS_BLK + j) * x1[j];
+                    for (int n = 0; n < NE; n++) {
+                        acc[n] = acc[n] + p[n][j];
+                        pn[n][j] = weight(kn, n, bn * RS_BLK + j) * x1[j];
+                    }
+                    if (j == 0) {
+                        issue_order();
+                        if (bl + 2 == BPC) {
+                            // this chunk's reads have returned, and the next
+                            // chunk has landed: loads issued after it stay
+                            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+                            wait_vm<NE + (RS_NB - 2) * PER>();
+                            bar();
+                            issue_order();
+                        }
+                        read(kr, br, x2);
+                    }
+                    // the chunk four ahead into this one's buffer, its
+                    // weights behind it into this one's registers
+                    if (bl >= BPC - 2 && (j == 4 || j == 10)) {
+                        issue_order();
+                        stage_k(k, c + k + RS_NB, 2 * (bl - (BPC - 2)) + (j == 10));
+                    }
+                    if (bl == BPC - 1 && j == 12) {
+                        issue_order();
+                        load_w(k, c + k + RS_NB);
+                    }
+                    issue_order();
+                }
+#pragma unroll
+                for (int j = 0; j < RS_BLK; j++) {
+                    x1[j] = x2[j];
+#pragma unroll
+                    for (int n = 0; n < NE; n++) p[n][j] = pn[n][j];
+                }
             }
-            if (j == 0 && blk + 2 < NBK) {
-                __builtin_amdgcn_sched_barrier(0);
-                rs_load_x(xrow, sw, blk + 2, x2);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int j = 0; j < RS_BLK; j++) {
-            x1[j] = x2[j];
-#pragma unroll
-            for (int n = 0; n < NE; n++) p[n][j] = pn[n][j];
-        }
-    }
-}
-
-// The chunk loop of one wave (work: the wave sums at all; gate: it sums the
-// gate; every wave stages and passes the same barriers).  Per chunk c: take
-// the weights loaded during chunk c - 1, issue the direct-to-LDS batch of
-// chunk c + RS_NB - 1 and the weights of chunk c + 1, sum chunk c, then wait
-// for batch c + 1 and pass a barrier.  Waiting for batch c + 1 leaves in
-// flight what was issued after it: with four buffers the weights of chunks
-// c - 1 .. c + 1 (2 NE + 2 loads each) and batches c + 2 and c + 3 (RS_XI
-// each); with two, the weights of chunk c + 1.
-template <int NE>
-__device__ __forceinline__ void rs_run(RsSmem &S, const float *__restrict__ x, const float *w0,
-                                       const uint16_t *__restrict__ g, int t0, int T, int H, bool work, bool gate,
-                                       float (&acc)[NE])
-{
-    const int lane = lane_id(), wv = wave_id();
-    const int nc = H / RS_CJ;
-    constexpr int AFTER = 2 * RS_XI + 3 * (2 * NE + 2);
-    static_assert(RS_NB != 4 || AFTER < 64, "vmcnt range");
-    rs_f4 wn[NE][2], wc[NE][2];
-    uint2 gn[2];
-    for (int c = 0; c < RS_NB - 1 && c < nc; c++) rs_stage(S, c, x, w0, t0, T, H, c, wv, lane);
-    issue_order();
-    rs_load_w<NE>(wn, gn, w0, g, H, 0, lane);
-    wait_vm<0>();
-    bar();
-    for (int c = 0; c < nc; c++) {
-        rs_take<NE>(wc, wn, gn, gate);
-        // buffer (c + RS_NB - 1) % RS_NB was last read in chunk c - 1,
-        // before the barrier that ended it
-        if (c + RS_NB - 1 < nc)
-            rs_stage(S, (c + RS_NB - 1) % RS_NB, x, w0, t0, T, H, c + RS_NB - 1, wv, lane);
-        issue_order();
-        if (c + 1 < nc) rs_load_w<NE>(wn, gn, w0, g, H, c + 1, lane);
-        issue_order();
-        if (work) chunk_dot<NE>(S.x[c % RS_NB][lane], lane & 15, wc, acc);
-        if (c + 1 < nc) {
-            if constexpr (RS_NB == 4) {
-                if (c + 3 < nc) wait_vm<AFTER>();
-                else wait_vm<0>();
-            } else {
-                static_assert(RS_NB == 2, "chunk buffers");
-                wait_vm<2 * NE + 2>();  // chunk c + 1's weights were issued after its batch
-            }
-            bar();
         }
     }
+    wait_vm<0>();  // (the loads past the end)
 }
 
 // Workgroup (bx, by) of a grid (nbx + shg_row, ceil(T / 64)) of 256
 // threads, nbx = ceil(E / (4 NE)): router rows 4 NE bx .. + 4 NE - 1 (NE a
 // wave) for tokens 64 by .. (one a lane); with shg_row, workgroup bx = nbx
-// takes the fp16 shared gate (on wave 0; written to gsh, 0 when shg is NULL).
-// H % 128 == 0 and E >= NE.
+// takes the fp16 shared gate (written to gsh by wave 0, 0 when shg is NULL).
+// H % 256 == 0 and E >= NE.
 template <int NE>
-__device__ __forceinline__ void route_seq_block(RsSmem &S, int bx, int by, const float *__restrict__ router,
-                                                const uint16_t *__restrict__ shg, const float *__restrict__ x,
-                                                float *__restrict__ logits, float *__restrict__ gsh, int H, int E,
-                                                int T, bool shg_row)
+__device__ __forceinline__ void route_seq_block(RsBuf &b0, RsBuf &b1, RsBuf &b2, RsBuf &b3, int bx, int by,
+                                                const float *__restrict__ router, const uint16_t *__restrict__ shg,
+                                                const float *__restrict__ x, float *__restrict__ logits,
+                                                float *__restrict__ gsh, int H, int E, int T, bool shg_row)
 {
-    static_assert(NE == 1 || NE == 2, "weight registers");
     const int lane = lane_id(), wv = wave_id();
     const int nbx = (E + RS_WAVES * NE - 1) / (RS_WAVES * NE);
-    const bool gate_wg = shg_row && bx == nbx;
-    const bool gate_wave = gate_wg && wv == 0 && shg;  // sums the gate
-    const int t0 = by * RS_TT;
+    const int t0 = by * RS_TT, t = t0 + lane, nt = min(RS_TT, T - t0);
+    const float *xt = x + (size_t)t0 * H;
+    if (shg_row && bx == nbx) {
+        float acc[1] = {0.f};
+        if (shg) rs_run<1, true>(b0, b1, b2, b3, xt, nt, nullptr, shg, H, acc);
+        if (wv == 0 && t < T) gsh[t] = acc[0];
+        return;
+    }
     // the wave stands for rows eb .. eb + NE - 1 and sums the NE consecutive
     // rows from e0 (moved back from eb so that every row read exists; rows
-    // past E are not stored); the gate workgroup's waves read row 0
+    // past E are not stored)
     const int eb = bx * RS_WAVES * NE + wv * NE;
-    const int e0 = gate_wg ? 0 : min(eb, E - NE);
-    const float *w0 = router + (size_t)e0 * H;
+    const int e0 = min(eb, E - NE);
     float acc[NE];
 #pragma unroll
     for (int n = 0; n < NE; n++) acc[n] = 0.f;
-    const uint16_t *g = shg ? shg : reinterpret_cast<const uint16_t *>(w0);
-    rs_run<NE>(S, x, w0, g, t0, T, H, !gate_wg || gate_wave, gate_wave, acc);
-    const int t = t0 + lane;
+    rs_run<NE, false>(b0, b1, b2, b3, xt, nt, router + (size_t)e0 * H, nullptr, H, acc);
     if (t >= T) return;
-    if (gate_wg) {
-        if (wv == 0) gsh[t] = shg ? acc[0] : 0.f;
-        return;
-    }
 #pragma unroll
     for (int n = 0; n < NE; n++) {
         const int e = e0 + n;
