@@ -304,6 +304,11 @@ __global__ __launch_bounds__(256) void k_gateup(bread_moe_layer_t L, const float
 // One wave per (token, output row): down rows of every slot, combined in the
 // reference order (one_layer.cu:1447-1469): the shared expert (when
 // `shared`), then the routed experts by rank.
+// Latency bound: 16 MB of weights over 2048 waves a token.  A superblock is
+// eight lanes' work, so a row of 512 columns would leave 48 of 64 lanes idle,
+// and the slots one after another wait for memory each; the wave takes eight
+// (slot, superblock) pairs at once instead, two passes in flight, and sums
+// them in slot order.  One token, 8 slots of 512: 15.4 -> 7.2 us on MI355X.
 __global__ __launch_bounds__(256) void k_down(bread_moe_layer_t L, const int32_t *__restrict__ idx,
                                               const float *__restrict__ w, const float *__restrict__ gsh,
                                               const float *__restrict__ h, float *__restrict__ hidden, int H,
@@ -324,12 +329,32 @@ __global__ __launch_bounds__(256) void k_down(bread_moe_layer_t L, const int32_t
             st, (const uint8_t *)L.down_shexp + (uint64_t)r * bread_expert_row_bytes(st, Ish), Ish / QK, ht, lane));
         acc += sigmoidf_ref(gsh[t]) * sh;
     }
-    const uint64_t rb = bread_expert_row_bytes(dt, I);
-    for (int k = 0; k < K; k++) {
+    const int nb = I / QK, np = K * nb;
+    const uint32_t bb = (uint32_t)bread_expert_row_bytes(dt, QK);
+    // the lane's eighth of pair q (slot q / nb, superblock q % nb; past the
+    // end the last one, which the sums leave out), summed over its eight lanes
+    auto pair = [&](int q) __attribute__((always_inline)) {
+        q = min(q, np - 1);
+        const int k = q / nb, b = q - k * nb;
         const int e = checked_expert(idx[(size_t)t * K + k], E, err);
-        const uint8_t *d = (const uint8_t *)L.down_exps + (uint64_t)e * L.down_expert_bytes + r * rb;
-        const float eo = wave_sum(kq_row_partial(dt, d, I / QK, ht + (size_t)(k + 1) * Imax, lane));
-        acc += w[(size_t)t * K + k] * eo;
+        const uint8_t *d = (const uint8_t *)L.down_exps + (uint64_t)e * L.down_expert_bytes +
+                           ((uint64_t)r * nb + b) * bb;
+        return sum8(kq_row_partial(dt, d, 1, ht + (size_t)(k + 1) * Imax + b * QK, lane & 7));
+    };
+    float eo = 0.f;
+    int k = 0, b = 0;
+    for (int q = 0; q < np; q += 16) {
+        const float v0 = pair(q + (lane >> 3)), v1 = pair(q + 8 + (lane >> 3));
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            eo += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, i < 8 ? v0 : v1), 8 * (i & 7)));
+            if (++b == nb) {
+                if (k < K) acc += w[(size_t)t * K + k] * eo;
+                eo = 0.f;
+                b = 0;
+                k++;
+            }
+        }
     }
     if (lane == 0) hidden[(size_t)t * H + r] = acc;
 }
@@ -549,18 +574,18 @@ extern "C" int bread_stack_loop_tokens(void)
 // an expert's rows once for every token that chose it.  us a layer on MI355X
 // (hidden 2048, intermediate 512, 256 experts, top 8, uniform routing),
 // per-token / grouped:
-//   tokens               2          3         4          6          8         27         130
-//   all Q4_K           61 / 68   78 / 70   88 / 71   120 / 75   151 / 79   421 / 146  1765 / 206
-//   all Q6_K           61 / 102  79 / 110  95 / 112  131 / 116  165 / 120  451 / 236  1886 / 360
-//   Q6_K shared down   60 / 85   77 / 87   87 / 89   119 / 93   152 / 99   423 / 163  1774 / 225
-// (Q6_K gate and up weights are gathered a row a lane; a shared expert of
-// another type takes launches of its own).
+//   tokens               4          5         8          10         27         130
+//   all Q4_K           66 / 70   73 / 73   105 / 80   121 / 104  272 / 145  1137 / 201
+//   Q6_K shared down   65 / 88   73 / 89   105 / 99   122 / 123  274 / 162  1150 / 222
+//   all Q6_K           68 / 111  78 / 112  112 / 118  130 / 168  289 / 235  1195 / 359
+// (a shared expert of another type takes launches of its own; Q6_K gate and
+// up weights are gathered a row a lane.)
 static bool grouped_takes_mix(const bread_moe_layer_t *L, int T, const float *hidden)
 {
     const int Q4 = BREAD_QTYPE_Q4_K;
-    const bool all_q4 = L->gate_type == Q4 && L->up_type == Q4 && L->down_type == Q4 && L->gate_shexp_type == Q4 &&
-                        L->up_shexp_type == Q4 && L->down_shexp_type == Q4;
-    return T >= (all_q4 ? 3 : 6) && ((uintptr_t)hidden & 15) == 0;
+    const bool gu_q4 = L->gate_type == Q4 && L->up_type == Q4 && L->gate_shexp_type == Q4 && L->up_shexp_type == Q4;
+    const bool dn_q4 = L->down_type == Q4 && L->down_shexp_type == Q4;
+    return T >= (!gu_q4 ? 16 : dn_q4 ? 5 : 8) && ((uintptr_t)hidden & 15) == 0;
 }
 
 extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L, const float *x, float *hidden,
