@@ -265,16 +265,37 @@ __global__ __launch_bounds__(1024) void k_mt_bucket(const int32_t *__restrict__ 
                                                     int *__restrict__ pair_tok, int *__restrict__ pos_of,
                                                     MtTile *__restrict__ tiles, int *__restrict__ n_tiles)
 {
-    __shared__ int cnt[1024], base[1024], cur[1024];
+    __shared__ int cnt[1024], base[1024];
     __shared__ int wsa[16], wsb[16];
     const int tid = threadIdx.x;
     cnt[tid] = 0;
-    cur[tid] = 0;
     __syncthreads();
     const int P = T * K;
-    for (int p = tid; p < P; p += 1024) {
-        const int e = idx[p];
-        if ((unsigned)e < (unsigned)E) atomicAdd(&cnt[e], 1);
+    // PB pairs a thread and pass, an LDS atomic each: its count so far is the
+    // pair's place in its expert's list.  The first pass stays in registers,
+    // later ones leave the place in pos_of for the second walk.  (A pair at a
+    // time, with a second atomic in the second walk, each pair waited for
+    // memory twice: 2048 tokens 22 us, now 16 us.)
+    constexpr int PB = 16;
+    int e[PB], o[PB];
+    auto load = [&](int p0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            const int p = p0 + i * 1024 + tid;
+            e[i] = p < P ? idx[p] : -1;
+        }
+    };
+    for (int p0 = (P - 1) / (PB * 1024) * (PB * 1024); p0 >= 0; p0 -= PB * 1024) {
+        load(p0);
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            o[i] = 0;
+            if ((unsigned)e[i] < (unsigned)E) o[i] = atomicAdd(&cnt[e[i]], 1);
+        }
+        if (p0 == 0) break;
+#pragma unroll
+        for (int i = 0; i < PB; i++)
+            if (p0 + i * 1024 + tid < P) pos_of[p0 + i * 1024 + tid] = o[i];
     }
     __syncthreads();
     const int c = tid < E ? cnt[tid] : 0;
@@ -283,14 +304,23 @@ __global__ __launch_bounds__(1024) void k_mt_bucket(const int32_t *__restrict__ 
     block_scan2(c, nt, wsa, wsb, xc, xt, tc, tt);
     base[tid] = xc;
     __syncthreads();
-    for (int p = tid; p < P; p += 1024) {
-        const int e = idx[p];
-        int pos = -1;
-        if ((unsigned)e < (unsigned)E) {
-            pos = base[e] + atomicAdd(&cur[e], 1);
-            pair_tok[pos] = p / K;
+    for (int p0 = 0; p0 < P; p0 += PB * 1024) {
+        if (p0) {
+            load(p0);
+#pragma unroll
+            for (int i = 0; i < PB; i++) o[i] = p0 + i * 1024 + tid < P ? pos_of[p0 + i * 1024 + tid] : 0;
         }
-        pos_of[p] = pos;
+#pragma unroll
+        for (int i = 0; i < PB; i++) {
+            const int p = p0 + i * 1024 + tid;
+            if (p >= P) break;
+            int pos = -1;
+            if ((unsigned)e[i] < (unsigned)E) {
+                pos = base[e[i]] + o[i];
+                pair_tok[pos] = p / K;
+            }
+            pos_of[p] = pos;
+        }
     }
     for (int i = 0; i < nt; i++) tiles[xt + i] = {tid, xc + i * MT, min(MT, c - i * MT), 0};
     const int nsh = (T + MT - 1) / MT;
