@@ -263,6 +263,29 @@ __device__ __forceinline__ int checked_expert(int e, int E, uint32_t *err)
     return e < 0 ? 0 : E - 1;
 }
 
+// Two Q4_K rows against the same x, the loads of both in flight together
+// (a second row's loads after the first one's dot: one token, 8 slots of 512
+// rows of 2048 columns 9.0 us on MI355X, now 7.0); each sum as
+// q4k_row_partial's.
+__device__ __forceinline__ void q4k_row_pair_partial(const uint8_t *g, const uint8_t *u, int nb, const float *x,
+                                                     int lane, float &gv, float &uv)
+{
+    const int c = lane & 7;
+    const uint32_t j = (uint32_t)c >> 1;
+    gv = uv = 0.f;
+    for (int b = lane >> 3; b < nb; b += 8) {
+        const size_t o = (size_t)b * Q4K_BYTES;
+        const uint4 gh = ld_b128(g + o), uh = ld_b128(u + o);
+        const uint4 gq = ld_b128(g + o + 16 + 16 * c), uq = ld_b128(u + o + 16 + 16 * c);
+        float xl[16], xh[16];
+        const int base = b * QK + 64 * (int)j + 16 * (c & 1);
+        load_x16(x, base, xl);
+        load_x16(x, base + 32, xh);
+        gv += q4k_chunk_dot(gh, gq, j, xl, xh);
+        uv += q4k_chunk_dot(uh, uq, j, xl, xh);
+    }
+}
+
 // One wave per (token, slot, row): gate and up rows, then SwiGLU.  Each
 // tensor has its own type (Q4_K or Q6_K), as in the reference's
 // cpu_tensor_matvec dispatch (one_layer.cu:1465-1468).  Slot 0 (the shared
@@ -296,8 +319,17 @@ __global__ __launch_bounds__(256) void k_gateup(bread_moe_layer_t L, const float
     }
     const float *xt = x + (size_t)t * H;
     const int lane = lane_id();
-    const float gv = wave_sum(kq_row_partial(gt, g + r * bread_expert_row_bytes(gt, H), H / QK, xt, lane));
-    const float uv = wave_sum(kq_row_partial(ut, u + r * bread_expert_row_bytes(ut, H), H / QK, xt, lane));
+    g += r * bread_expert_row_bytes(gt, H);
+    u += r * bread_expert_row_bytes(ut, H);
+    float gv, uv;
+    if (gt == BREAD_QTYPE_Q4_K && ut == BREAD_QTYPE_Q4_K) {
+        q4k_row_pair_partial(g, u, H / QK, xt, lane, gv, uv);
+    } else {
+        gv = kq_row_partial(gt, g, H / QK, xt, lane);
+        uv = kq_row_partial(ut, u, H / QK, xt, lane);
+    }
+    gv = wave_sum(gv);
+    uv = wave_sum(uv);
     if (lane == 0) h[((size_t)t * (K + 1) + slot) * Imax + r] = silu_mul(gv, uv);
 }
 
@@ -574,10 +606,10 @@ extern "C" int bread_stack_loop_tokens(void)
 // an expert's rows once for every token that chose it.  us a layer on MI355X
 // (hidden 2048, intermediate 512, 256 experts, top 8, uniform routing),
 // per-token / grouped:
-//   tokens               4          5         8          10         27         130
-//   all Q4_K           66 / 70   73 / 73   105 / 80   121 / 104  272 / 145  1137 / 201
-//   Q6_K shared down   65 / 88   73 / 89   105 / 99   122 / 123  274 / 162  1150 / 222
-//   all Q6_K           68 / 111  78 / 112  112 / 118  130 / 168  289 / 235  1195 / 359
+//   tokens               5          6         10         16         27        130
+//   all Q4_K           67 / 73   77 / 73   110 / 104  157 / 111  242 / 145   993 / 201
+//   Q6_K shared down   66 / 89   77 / 92   111 / 123  159 / 129  245 / 162  1004 / 222
+//   all Q6_K           78 / 112  92 / 115  130 / 168  188 / 177  289 / 235  1194 / 359
 // (a shared expert of another type takes launches of its own; Q6_K gate and
 // up weights are gathered a row a lane.)
 static bool grouped_takes_mix(const bread_moe_layer_t *L, int T, const float *hidden)
@@ -585,7 +617,7 @@ static bool grouped_takes_mix(const bread_moe_layer_t *L, int T, const float *hi
     const int Q4 = BREAD_QTYPE_Q4_K;
     const bool gu_q4 = L->gate_type == Q4 && L->up_type == Q4 && L->gate_shexp_type == Q4 && L->up_shexp_type == Q4;
     const bool dn_q4 = L->down_type == Q4 && L->down_shexp_type == Q4;
-    return T >= (!gu_q4 ? 16 : dn_q4 ? 5 : 8) && ((uintptr_t)hidden & 15) == 0;
+    return T >= (!gu_q4 ? 16 : dn_q4 ? 6 : 12) && ((uintptr_t)hidden & 15) == 0;
 }
 
 extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L, const float *x, float *hidden,

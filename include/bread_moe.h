@@ -270,8 +270,8 @@ int bread_route_layer_f16(bread_moe_ctx_t *ctx, const bread_moe_layer_t *layer, 
  * grouped path (tokens bucketed by expert, expert GEMMs on the matrix cores
  * with fp16 operands and fp32 accumulation; intermediate sizes <= 512 and
  * 16-byte aligned Q6_K down weights); other shapes run the per-token path.
- * Other weight-type mixes run the grouped path from a few tokens on (5 where
- * every tensor is Q4_K, 8 where every gate and up is, 16 otherwise; shapes and
+ * Other weight-type mixes run the grouped path from a few tokens on (6 where
+ * every tensor is Q4_K, 12 where every gate and up is, 16 otherwise; shapes and
  * alignment as above, d_hidden 16-byte aligned) with operands that keep
  * fp32's precision, and the per-token path else.  A pinned path that does not take the layer's weight
  * types returns BREAD_ERR_QTYPE. */

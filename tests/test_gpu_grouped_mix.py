@@ -1,6 +1,6 @@
 """Layers of other mixes of Q4_K and Q6_K than the decode kernel's under the
 automatic choice, around the token counts where it moves from the per-token
-kernels to the grouped path (5 with every tensor Q4_K, 8 with every gate and
+kernels to the grouped path (6 with every tensor Q4_K, 12 with every gate and
 up tensor Q4_K, 16 otherwise), for each tensor Q6_K by itself, and where the grouped path does not take the call
 (Q6_K down weights or the residual 4-byte aligned only).
 
@@ -34,7 +34,7 @@ def run(s, d, x, hidden, path):
     return hidden.cpu().numpy(), idx.cpu().numpy(), w.cpu().numpy(), g.cpu().numpy()
 
 
-@pytest.mark.parametrize("T", [2, 5, 8, 16, 33])
+@pytest.mark.parametrize("T", [5, 6, 12, 16, 33])
 @pytest.mark.parametrize("mix", MIXES)
 @pytest.mark.parametrize("H,I,Ish,off", [(768, 256, 512, 0), (512, 512, 512, 0), (512, 512, 512, 1)])
 def test_mix_auto_matches_per_token(mix, T, H, I, Ish, off):
