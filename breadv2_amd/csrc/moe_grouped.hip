@@ -583,22 +583,6 @@ struct Unit<BREAD_QTYPE_Q6_K, X> {
     }
 };
 
-// silu(g) * u (layer_ops.cu:214-220): exp from the hardware's exp2 with the
-// rounding of g log2(e) added back, the quotient by Newton steps on the
-// hardware reciprocal; exact division where that could overflow.
-__device__ __forceinline__ float swiglu(float g, float u)
-{
-    const float t = -1.44269504088896f * g;
-    const float lo = fmaf(-1.44269504088896f, g, -t) + g * -1.925963033500e-8f;  // t's rounding, log2(e)'s
-    const float e = __builtin_amdgcn_exp2f(t);
-    const float den = 1.0f + (fabsf(t) < 128.f ? fmaf(e, 0.693147180559945f * lo, e) : e);
-    float q = __builtin_amdgcn_rcpf(den);
-    q = fmaf(fmaf(-den, q, 1.0f), q, q);
-    float v = g * q;
-    v = fmaf(fmaf(-den, v, g), q, v);
-    return (den < 1e30f ? v : g / den) * u;
-}
-
 struct GgArgs {
     const uint8_t *w0, *w1;    // routed gate and up (or down), expert e at + e * stride
     uint64_t st0, st1;
@@ -922,7 +906,7 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
         for (int i = 0; i < 16; i++) {
             const int n = 8 * (i >> 2) + 4 * g + (i & 3);
             const int ex = sexp[turn][n];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, swiglu(ldexpf(t0[i], ex), ldexpf(t1[i], ex))),
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, silu_mul(ldexpf(t0[i], ex), ldexpf(t1[i], ex))),
                                                   hb, 4 * (uint32_t)(n * a.hstride) + 4 * col, 0, 0);
         }
         if (!more) break;
