@@ -11,13 +11,18 @@
 // Numerics.  MFMA operands are fp16 with fp32 accumulation, and every
 // product is exact.  A weight enters as its integer part: sc * q (Q4_K,
 // <= 63 * 15) or sc * (q - 32) (Q6_K, |.| <= 4096: exact up to 2048 and for
-// even values; the odd ones above are rounded to even in layers of the
-// reference GPU path's types and carried by a second operand in the others,
-// which keep fp32's precision), times a power of two.  Activations are two fp16 terms (hi + lo, 22
-// significant bits) after a power-of-two row scale into [2^13, 2^14) (exact,
-// undone on the fp32 result).  The superblock scale d, and for Q4_K the min
-// term dmin * sum_j m_j * (sum of x over sub-block j), are applied to the
-// fp32 sums.
+// even values), times a power of two.  Activations are two fp16 terms (hi +
+// lo, 23 significant bits at most) after a power-of-two row scale into
+// [2^13, 2^14) (exact, undone on the fp32 result).  The superblock scale d,
+// and for Q4_K the min term dmin * sum_j m_j * (sum of x over sub-block j),
+// are applied to the fp32 sums.
+// Layers of the reference GPU path's types round the odd Q6_K integers above
+// 2048 to even (7e-5 of a layer's output).  Layers of other types (X), which
+// run in fp32 at fewer tokens, carry that rest in a second operand and scale
+// the lo terms (LO_EXP): their inputs are off by 2^-23 at most, and with exact
+// products the sums come out as near to 64-bit arithmetic as the per-token
+// kernels' (27 tokens of hidden 2048, all Q4_K: 5.5e-7 both, all Q6_K: 2.6e-7
+// both).
 //
 // Kernels per layer, stream-ordered:
 //   k_route_seq   router logits in the reference's sequential order
@@ -84,11 +89,22 @@ __device__ __forceinline__ int row_exp(float max_abs)
     return e;
 }
 
-// v (already scaled) as hi + lo fp16: hi = fp16(v), lo = fp16(v - hi).
-__device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t &lo)
+// The lo terms of layers of other types than the reference GPU path's (X
+// below) are held times 2^LO_EXP.  A lo term then has its 11 bits wherever the
+// hi term has, so a value keeps 23 bits down to 2^-24 of its row's largest;
+// unscaled, it runs into the end of fp16's subnormals from 2^-14 on, and a
+// channel 10^5 or 10^7 times the others left the rest of a row errors of
+// 1.5e-7 or 1.6e-5.  The weights that meet lo terms are times 2^-LO_EXP: 2^10
+// is the most at which a Q4_K one (an integer times 2^-14) is an fp16 number.
+// The lo terms of the sub-block sums meet integers alone and are held times
+// 2^SUM_LO_EXP, the most that fits fp16.
+constexpr int LO_EXP = 10, SUM_LO_EXP = 13;
+
+// v (already scaled) as hi + lo / ls fp16: hi = fp16(v), lo = fp16((v - hi) ls).
+__device__ __forceinline__ void split2(float a, float b, float ls, uint32_t &hi, uint32_t &lo)
 {
     const _Float16 ha = (_Float16)a, hb = (_Float16)b;
-    const _Float16 la = (_Float16)(a - (float)ha), lb = (_Float16)(b - (float)hb);
+    const _Float16 la = (_Float16)((a - (float)ha) * ls), lb = (_Float16)((b - (float)hb) * ls);
     hi = (uint32_t)__builtin_bit_cast(uint16_t, ha) | ((uint32_t)__builtin_bit_cast(uint16_t, hb) << 16);
     lo = (uint32_t)__builtin_bit_cast(uint16_t, la) | ((uint32_t)__builtin_bit_cast(uint16_t, lb) << 16);
 }
@@ -116,21 +132,21 @@ __device__ __forceinline__ int unit_base(int u)
 
 // Eight elements in operand order (a: b .. b + 3, c: b + 32 .. b + 35),
 // scaled by 2^-e and split.
-__device__ __forceinline__ void split_unit(const float4 &a, const float4 &c, int e, uint4 &hi, uint4 &lo)
+__device__ __forceinline__ void split_unit(const float4 &a, const float4 &c, int e, float ls, uint4 &hi, uint4 &lo)
 {
-    split2(ldexpf(a.x, -e), ldexpf(a.z, -e), hi.x, lo.x);
-    split2(ldexpf(a.y, -e), ldexpf(a.w, -e), hi.y, lo.y);
-    split2(ldexpf(c.x, -e), ldexpf(c.z, -e), hi.z, lo.z);
-    split2(ldexpf(c.y, -e), ldexpf(c.w, -e), hi.w, lo.w);
+    split2(ldexpf(a.x, -e), ldexpf(a.z, -e), ls, hi.x, lo.x);
+    split2(ldexpf(a.y, -e), ldexpf(a.w, -e), ls, hi.y, lo.y);
+    split2(ldexpf(c.x, -e), ldexpf(c.z, -e), ls, hi.z, lo.z);
+    split2(ldexpf(c.y, -e), ldexpf(c.w, -e), ls, hi.w, lo.w);
 }
 
 // The same for eight elements already in operand order.
-__device__ __forceinline__ void split_unit_op(const float4 &a, const float4 &c, int e, uint4 &hi, uint4 &lo)
+__device__ __forceinline__ void split_unit_op(const float4 &a, const float4 &c, int e, float ls, uint4 &hi, uint4 &lo)
 {
-    split2(ldexpf(a.x, -e), ldexpf(a.y, -e), hi.x, lo.x);
-    split2(ldexpf(a.z, -e), ldexpf(a.w, -e), hi.y, lo.y);
-    split2(ldexpf(c.x, -e), ldexpf(c.y, -e), hi.z, lo.z);
-    split2(ldexpf(c.z, -e), ldexpf(c.w, -e), hi.w, lo.w);
+    split2(ldexpf(a.x, -e), ldexpf(a.y, -e), ls, hi.x, lo.x);
+    split2(ldexpf(a.z, -e), ldexpf(a.w, -e), ls, hi.y, lo.y);
+    split2(ldexpf(c.x, -e), ldexpf(c.y, -e), ls, hi.z, lo.z);
+    split2(ldexpf(c.z, -e), ldexpf(c.w, -e), ls, hi.w, lo.w);
 }
 
 // ---------------------------------------------------------------------------
@@ -146,10 +162,11 @@ __device__ __forceinline__ float xor_add(float v, int m)
 }
 
 __device__ __forceinline__ void mt_xprep(int t, const float *__restrict__ x, const uint16_t *__restrict__ shg, int H,
-                                         uint4 *__restrict__ xop, uint4 *__restrict__ xsum, int *__restrict__ xexp,
-                                         float *__restrict__ gsh)
+                                         bool scaled_lo, uint4 *__restrict__ xop, uint4 *__restrict__ xsum,
+                                         int *__restrict__ xexp, float *__restrict__ gsh)
 {
     __shared__ float smax[4], sdot[4];
+    const float ls = scaled_lo ? (float)(1 << LO_EXP) : 1.f, ls_sum = scaled_lo ? (float)(1 << SUM_LO_EXP) : 1.f;
     const float *xt = x + (size_t)t * H;
     float mx = 0.f, dot = 0.f;
     for (int i = 4 * (int)threadIdx.x; i < H; i += 1024) {
@@ -183,7 +200,7 @@ __device__ __forceinline__ void mt_xprep(int t, const float *__restrict__ x, con
         const float4 a = *reinterpret_cast<const float4 *>(xt + b);
         const float4 c = *reinterpret_cast<const float4 *>(xt + b + 32);
         uint4 h, l;
-        split_unit(a, c, e, h, l);
+        split_unit(a, c, e, ls, h, l);
         uint4 *o = xop + ((size_t)t * (H / QK) + sb) * 64;
         o[u & 31] = h;
         o[32 + (u & 31)] = l;
@@ -193,7 +210,7 @@ __device__ __forceinline__ void mt_xprep(int t, const float *__restrict__ x, con
         sc = xor_add(xor_add(xor_add(sc, 2), 4), 8);
         if ((u & 0xE) == 0) {
             uint32_t hh, ll;
-            split2(sa, sc, hh, ll);
+            split2(sa, sc, ls_sum, hh, ll);
             uint32_t *so = reinterpret_cast<uint32_t *>(xsum + ((size_t)t * (H / QK) + sb) * 2);
             const int j2 = 2 * (u & 1) + ((u >> 4) & 1);  // j / 2
             so[j2] = hh;
@@ -210,8 +227,9 @@ template <int MAXV>
 __global__ __launch_bounds__(256) void k_mt_topk_xprep(const float *__restrict__ logits, int E, int K,
                                                        int32_t *__restrict__ idx, float *__restrict__ w,
                                                        const float *__restrict__ x, const uint16_t *__restrict__ shg,
-                                                       int H, uint4 *__restrict__ xop, uint4 *__restrict__ xsum,
-                                                       int *__restrict__ xexp, float *__restrict__ gsh)
+                                                       int H, bool scaled_lo, uint4 *__restrict__ xop,
+                                                       uint4 *__restrict__ xsum, int *__restrict__ xexp,
+                                                       float *__restrict__ gsh)
 {
     __shared__ __attribute__((aligned(16))) float s_e[WAVE * MAXV];
     const int t = (int)blockIdx.x;
@@ -224,7 +242,7 @@ __global__ __launch_bounds__(256) void k_mt_topk_xprep(const float *__restrict__
             w[(size_t)t * K + lane_id()] = wk;
         }
     }
-    mt_xprep(t, x, shg, H, xop, xsum, xexp, gsh);
+    mt_xprep(t, x, shg, H, scaled_lo, xop, xsum, xexp, gsh);
 }
 
 // ---------------------------------------------------------------------------
@@ -440,6 +458,14 @@ __device__ __forceinline__ half2v pair_u8(uint32_t v)
     return h2_of(__builtin_amdgcn_perm(0x64646464u, v, 0x07000700u | I | (J << 16))) - pair(1024.f, 1024.f);
 }
 
+// w 2^-EXP: eight weights for lo terms held times 2^EXP.
+template <int EXP>
+__device__ __forceinline__ uint4 lo_operand(const uint4 &w)
+{
+    const half2v k = pair(1.f / (1 << EXP), 1.f / (1 << EXP));
+    return make_uint4(u_of(h2_of(w.x) * k), u_of(h2_of(w.y) * k), u_of(h2_of(w.z) * k), u_of(h2_of(w.w) * k));
+}
+
 // Operand maker of one unit (32 weight rows of one superblock): constants
 // from the superblock's header, then a step's eight weights; the scaling of
 // the sums.  prepare() sets bad when the superblock is outside the range that
@@ -476,13 +502,14 @@ struct Unit<BREAD_QTYPE_Q4_K, X> {
     // tot += 2^14 d c - sum_j dmin m_j (sum of x over sub-block j), with X +
     // sum_j 8 d sc_j of them: m_0..7 and sc_0..7 against the hi and lo sums.
     // The last two are of one size and cancel, so they meet before the total.
-    __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q4_K> &R, const uint4 &sums, const f32x16 &c,
+    __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q4_K> &R, const uint4 &sums, int g, const f32x16 &c,
                                         f32x16 &tot) const
     {
         const uint32_t s0 = R.hd.y, s1 = R.hd.z, s2 = R.hd.w;
-        auto eight = [](uint32_t lo, uint32_t hi) __attribute__((always_inline)) {
-            return make_uint4(u_of(pair_u8<0, 1>(lo)), u_of(pair_u8<2, 3>(lo)), u_of(pair_u8<0, 1>(hi)),
-                              u_of(pair_u8<2, 3>(hi)));
+        auto eight = [g](uint32_t lo, uint32_t hi) __attribute__((always_inline)) {
+            const uint4 v = make_uint4(u_of(pair_u8<0, 1>(lo)), u_of(pair_u8<2, 3>(lo)), u_of(pair_u8<0, 1>(hi)),
+                                       u_of(pair_u8<2, 3>(hi)));
+            return X && g ? lo_operand<SUM_LO_EXP>(v) : v;  // lane half 1 meets the lo sums
         };
         const uint4 mv = eight(s1 & 0x3F3F3F3Fu, ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u));
         const f32x16 pm = mfma32(sums, mv, zero16());
@@ -547,7 +574,7 @@ struct Unit<BREAD_QTYPE_Q6_K, X> {
         }
     }
 
-    __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q6_K> &R, const uint4 &, const f32x16 &c,
+    __device__ __forceinline__ void add(const Raw<BREAD_QTYPE_Q6_K> &R, const uint4 &, int, const f32x16 &c,
                                         f32x16 &tot) const
     {
         const float d = (X ? 1.f : 0x1p16f) * h2f(R.d);
@@ -824,10 +851,12 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
             }
             c0 = mfma32(xh, w0, c0);
             c1 = mfma32(xh, w1, c1);
-            c0 = mfma32(xl, w0, c0);
-            c1 = mfma32(xl, w1, c1);
+            c0 = mfma32(xl, X ? lo_operand<LO_EXP>(w0) : w0, c0);
+            c1 = mfma32(xl, X ? lo_operand<LO_EXP>(w1) : w1, c1);
             if (X0) c0 = mfma32(xh, r0, c0);
             if (X1) c1 = mfma32(xh, r1, c1);
+            if (X0) c0 = mfma32(xl, lo_operand<LO_EXP>(r0), c0);
+            if (X1) c1 = mfma32(xl, lo_operand<LO_EXP>(r1), c1);
             if (s < 7) {
                 U0.step(R0, C, 8 * pp + s + 1, v0, q0);
                 U1.step(R1, C, 8 * pp + s + 1, v1, q1);
@@ -835,9 +864,9 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
             // an MFMA, then VALU: the next step's operands are made under
             // this one's products
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < 4 + 2 * X0 + 2 * X1; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x2, X0 || X1 ? 14 : 5, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, X0 || X1 ? 10 : X ? 7 : 5, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
             xh = nh;
@@ -891,8 +920,8 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
             compute(sA1, 1);
             uint4 sums = make_uint4(0, 0, 0, 0);
             if (SUMS) sums = sS[r][g];
-            U0.add(R0, sums, c0, t0);
-            U1.add(R1, sums, c1, t1);
+            U0.add(R0, sums, g, c0, t0);
+            U1.add(R1, sums, g, c1, t1);
         }
         // SwiGLU, stored in operand order: row c of a superblock at its
         // unit's place (unit_base), for k_down_gg's loads
@@ -979,6 +1008,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K;
     constexpr bool X0 = X && QT != Q4;
+    constexpr float LS = X ? (float)(1 << LO_EXP) : 1.f;
     constexpr int NB = MAX_INTER / QK;
     __shared__ uint4 sA[NB][MT][64];
     __shared__ uint32_t sS[QT == Q4 ? NB : 1][MT][2][4];  // sums: hi, lo of eight
@@ -1047,7 +1077,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
             if (k >= 2 * nb) continue;
             const int b = k >> 1, u = hq + 16 * (k & 1);
             uint4 hi, lo;
-            split_unit_op(va[k], vb[k], ex, hi, lo);
+            split_unit_op(va[k], vb[k], ex, LS, hi, lo);
             sA[b][hn][u ^ (hn & 15)] = hi;
             sA[b][hn][32 + (u ^ (hn & 15))] = lo;
             if (QT == Q4) {
@@ -1060,7 +1090,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
                 sy = xor_add(xor_add(xor_add(sy, 2), 4), 8);
                 if (hq < 2) {
                     uint32_t h2, l2;
-                    split2(sx, sy, h2, l2);
+                    split2(sx, sy, X ? (float)(1 << SUM_LO_EXP) : 1.f, h2, l2);
                     sS[b][hn][0][2 * hq + (k & 1)] = h2;
                     sS[b][hn][1][2 * hq + (k & 1)] = l2;
                 }
@@ -1111,6 +1141,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
                 c0 = mfma32(xh, w0, c0);
                 c1 = mfma32(xl, w0, c1);
                 if (X0) c0 = mfma32(xh, r0, c0);
+                if (X0) c1 = mfma32(xl, r0, c1);
                 if (s < 15) U.step(R, C, s + 1, v0, q0);
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
@@ -1124,10 +1155,10 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
                 r0 = q0;
             }
 #pragma unroll
-            for (int i = 0; i < 16; i++) c0[i] += c1[i];
+            for (int i = 0; i < 16; i++) c0[i] = X ? fmaf(c1[i], 1.f / LS, c0[i]) : c0[i] + c1[i];
             uint4 sums = make_uint4(0, 0, 0, 0);
             if (QT == Q4) sums = *reinterpret_cast<const uint4 *>(sS[b][r][g]);
-            U.add(R, sums, c0, t);
+            U.add(R, sums, g, c0, t);
             if (b == nb - 1) {
                 // rows past nr (and blocks past the end) fall outside the
                 // buffer's range: every lane issues all 16 stores, which the
@@ -1296,10 +1327,10 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     }
     if (!standard) shg = nullptr;
     if ((E + WAVE - 1) / WAVE <= 4)
-        hipLaunchKernelGGL(k_mt_topk_xprep<4>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x, shg, H,
+        hipLaunchKernelGGL(k_mt_topk_xprep<4>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x, shg, H, !standard,
                            (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, gsh);
     else
-        hipLaunchKernelGGL(k_mt_topk_xprep<16>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x, shg, H,
+        hipLaunchKernelGGL(k_mt_topk_xprep<16>, dim3(T), dim3(256), 0, st, c->logits, E, K, c->idx, c->w, x, shg, H, !standard,
                            (uint4 *)g.xop, (uint4 *)g.xsum, g.xexp, gsh);
     BREAD_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_mt_bucket, dim3(1), dim3(1024), 0, st, c->idx, T, K, E, g.pair_tok, g.pos_of,

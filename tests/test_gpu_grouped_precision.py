@@ -14,6 +14,8 @@ import torch
 import breadv2_amd as B
 from breadv2_amd import api
 
+from helpers import rel_l2
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 Q4, Q6 = api.QTYPE_Q4_K, api.QTYPE_Q6_K
@@ -87,7 +89,7 @@ def run(t, x, path):
     T = x.shape[0]
     ctx = B.MoeContext(t.shape, max_tokens=T)
     ctx.set_path(path)
-    hd = torch.zeros(T, H, device=DEV)
+    hd = torch.zeros_like(x)
     ctx.forward(t.desc(), x, hd, T)
     torch.cuda.synchronize()
     assert ctx.check_device() == 0
@@ -95,15 +97,56 @@ def run(t, x, path):
 
 
 @pytest.mark.parametrize("T", [17, 130])
-@pytest.mark.parametrize("down_shared,path", [(Q6, api.PATH_GROUPED), (Q4, api.PATH_AUTO)])
-def test_swiglu_is_the_per_token_kernels(T, down_shared, path):
+@pytest.mark.parametrize("down_shared,path,tail", [(Q6, api.PATH_GROUPED, 2.0 ** -38), (Q4, api.PATH_AUTO, 2.0 ** -48)])
+def test_swiglu_is_the_per_token_kernels(T, down_shared, path, tail):
     """An output is its SwiGLU value in two fp16 terms: off by at most 2^-23 of
     itself (11 bits and 11 bits of the signed rest: half a unit of the second
-    term is 2^-23), or by 2^-38 of the row's largest, where the second term
-    meets the end of fp16's subnormals (2^-25 after a scale of 2^13)."""
+    term is 2^-23), or by what fp16's smallest number, 2^-24, leaves of a row
+    scaled to 2^13: half of it, and with the second term held times 2^10 (the
+    layers of other type mixes) a 2^-10th of that."""
     x = inputs(T)
     ref = run(layer((Q4, 1, 1), Q4), x, api.PATH_PER_TOKEN)
     got = run(layer((Q6, 1, 1), down_shared), x, path)
-    bound = 2.0 ** -23 * np.abs(ref) + 2.0 ** -38 * np.abs(ref).max(1, keepdims=True)
+    bound = 2.0 ** -23 * np.abs(ref) + tail * np.abs(ref).max(1, keepdims=True)
     assert np.count_nonzero(ref) == ref.size
     assert np.all(np.abs(got - ref) <= bound)
+
+
+@pytest.mark.parametrize("T", [17, 130])
+def test_q6k_weight_of_12_bits(T):
+    """A Q6_K weight of 127 * 31 = 3937, which fp16 rounds to an even integer,
+    in a layer of another type mix: the rest meets both terms of the SwiGLU
+    value, so what is off is the split (as above) and the rounding of the
+    terms' sum, 2^-24."""
+    x = inputs(T)
+    ref = 3937.0 * run(layer((Q4, 1, 1), Q4), x, api.PATH_PER_TOKEN)
+    got = run(layer((Q6, 127, 31), Q4), x, api.PATH_AUTO)
+    bound = (2.0 ** -23 + 2.0 ** -24) * np.abs(ref) + 2.0 ** -48 * np.abs(ref).max(1, keepdims=True)
+    assert np.all(np.abs(got - ref) <= bound)
+
+
+@pytest.mark.parametrize("typ", [Q4, Q6])
+@pytest.mark.parametrize("outlier", [1e3, 1e5, 1e7])
+def test_rows_with_an_outlier(typ, outlier):
+    """A channel far above the others that no gate, up or router row weighs
+    changes nothing but the row's scale, so the layer's output may move by the
+    splits of two operands, 2^-23 of a product each."""
+    H, T = 512, 24
+    s = api.shape(hidden=H, expert_inter=256, shared_inter=256, n_experts=12, top_k=3)
+    t = api.synth_layer_tensors(s, seed=5, layer=0, types=(typ,) * 6)
+    for name in ("gate_exps", "up_exps", "gate_sh", "up_sh"):  # columns 0..31 of each row
+        b = getattr(t, name).view(-1, H // 256, 144 if typ == Q4 else 210)
+        if typ == Q4:
+            b[:, 0, 4] &= 0xC0
+            b[:, 0, 8] &= 0xC0
+        else:
+            b[:, 0, 192:194] = 0
+    t.router.view(-1, H)[:, 0:32] = 0
+    t.shgate[0:32] = 0
+    x = torch.randn(T, H, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1))
+    out = []
+    for v, path in ((0.0, api.PATH_AUTO), (outlier, api.PATH_AUTO), (outlier, api.PATH_PER_TOKEN)):
+        x[:, 5] = v
+        out.append(run(t, x, path))
+    assert not np.array_equal(out[1], out[2])  # another path
+    assert rel_l2(out[1], out[0]) <= 2.0 ** -22
