@@ -602,22 +602,34 @@ extern "C" int bread_stack_loop_tokens(void)
 }
 
 // Whether a layer of another mix of Q4_K and Q6_K than the decode kernel's
-// goes to the grouped path rather than to the per-token kernels, which stream
-// an expert's rows once for every token that chose it.  us a layer on MI355X
-// (hidden 2048, intermediate 512, 256 experts, top 8, uniform routing),
-// per-token / grouped:
-//   tokens               5          6         10         16         27        130
-//   all Q4_K           67 / 73   77 / 73   110 / 104  157 / 111  242 / 145   993 / 201
-//   Q6_K shared down   66 / 89   77 / 92   111 / 123  159 / 129  245 / 162  1004 / 222
-//   all Q6_K           78 / 112  92 / 115  130 / 168  188 / 177  289 / 235  1194 / 359
-// (a shared expert of another type takes launches of its own; Q6_K gate and
-// up weights are gathered a row a lane.)
-static bool grouped_takes_mix(const bread_moe_layer_t *L, int T, const float *hidden)
+// goes to the grouped path rather than to the per-token kernels.  Those stream
+// an expert's rows once for every token that chose it, so their time grows by
+// the R = K I + Ish rows a token has; the grouped path's is flat for few tokens,
+// at its router, its launches and one tile's chain.  They meet at some number of
+// tokens T that the types set and, for smaller layers, at some T R (twice that
+// where the shared expert has a size of its own, hence launches of its own).
+// us a layer on MI355X, uniform routing, per-token / grouped:
+//   H, I, Ish, E, K           all Q4_K               Q6_K routed down          all Q6_K
+//   2048, 512, 512, 256, 8    6: 75 / 72             14: 128 / 129             16: 177 / 176
+//                             16: 144 / 106          20: 180 / 139             32: 327 / 244
+//   2048, 512, 512, 256, 2    8: 63 / 66, 10: 70 / 66    14: 86 / 86           16: 99 / 105, 20: 118 / 107
+//   1024, 512, 512, 64, 8     6: 53 / 51             12: 81 / 71               16: 117 / 75
+//   1024, 256, 512, 32, 4     16: 66 / 70, 20: 75 / 70   20: 73 / 74           24: 93 / 109, 32: 117 / 110
+//   768, 256, 512, 24, 4      16: 58 / 64, 20: 67 / 64   20: 66 / 68           24: 83 / 101, 32: 101 / 101
+//   512, 256, 256, 24, 4      10: 33 / 35, 12: 38 / 36   16: 44 / 47, 20: 49 / 47    16: 47 / 46
+//   256, 256, 256, 8, 2       16: 29 / 31, 20: 32 / 31   24: 37 / 43, 32: 44 / 42    20: 36 / 39, 24: 41 / 39
+//   4096, 512, 512, 128, 8    6: 119 / 118           12: 208 / 203             16: 342 / 316
+// (Q6_K gate and up weights are gathered a row a lane.)
+static bool grouped_takes_mix(const bread_moe_shape_t &s, const bread_moe_layer_t *L, int T, const float *hidden)
 {
     const int Q4 = BREAD_QTYPE_Q4_K;
     const bool gu_q4 = L->gate_type == Q4 && L->up_type == Q4 && L->gate_shexp_type == Q4 && L->up_shexp_type == Q4;
     const bool dn_q4 = L->down_type == Q4 && L->down_shexp_type == Q4;
-    return T >= (!gu_q4 ? 16 : dn_q4 ? 6 : 12) && ((uintptr_t)hidden & 15) == 0;
+    const bool one_size = s.expert_inter == s.shared_inter;
+    const int64_t rows = (int64_t)T * ((int64_t)s.top_k * s.expert_inter + s.shared_inter);
+    const int tokens = !gu_q4 ? 16 : dn_q4 ? 6 : 14;
+    const int least = !gu_q4 ? (one_size ? 30000 : 49000) : dn_q4 ? (one_size ? 15000 : 30000) : one_size ? 22000 : 33000;
+    return T >= tokens && rows >= least && ((uintptr_t)hidden & 15) == 0;
 }
 
 extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L, const float *x, float *hidden,
@@ -653,7 +665,7 @@ extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L,
     default:
         rc = (T == 1) ? bread_launch_moe_decode(c, L, x, hidden, st) : BREAD_ERR_SHAPE;
         if (rc == BREAD_ERR_SHAPE && T <= bread_small_auto_tokens()) rc = bread_launch_moe_small(c, L, x, hidden, T, st);
-        if (rc == BREAD_ERR_SHAPE && (bread_standard_qtypes(L) || grouped_takes_mix(L, T, hidden)))
+        if (rc == BREAD_ERR_SHAPE && (bread_standard_qtypes(L) || grouped_takes_mix(c->shape, L, T, hidden)))
             rc = bread_launch_moe_grouped(c, L, x, hidden, T, st);
         if (rc == BREAD_ERR_SHAPE) rc = bread_launch_moe_multi(c, L, x, hidden, T, st);
     }

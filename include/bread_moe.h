@@ -270,12 +270,12 @@ int bread_route_layer_f16(bread_moe_ctx_t *ctx, const bread_moe_layer_t *layer, 
  * grouped path (tokens bucketed by expert, expert GEMMs on the matrix cores
  * with fp16 operands and fp32 accumulation; intermediate sizes <= 512 and
  * 16-byte aligned Q6_K down weights); other shapes run the per-token path.
- * Other weight-type mixes run the grouped path from a few tokens on (6 where
- * every tensor is Q4_K, 12 where every gate and up is, 16 otherwise; shapes and
- * alignment as above, d_hidden 16-byte aligned) with operands of 23
- * bits (weights exact; as near to 64-bit sums as the per-token path), and the
- * per-token path else.  A pinned path that does not take the layer's weight
- * types returns BREAD_ERR_QTYPE. */
+ * Other weight-type mixes run the per-token path and, from some number of
+ * tokens on, the grouped one (6 where every tensor is Q4_K, 14 where every gate
+ * and up is, 16 otherwise, later for layers much smaller than the reference's;
+ * shapes and alignment as above, d_hidden 16-byte aligned), with operands of 23
+ * bits (weights exact; as near to 64-bit sums as the per-token path).  A pinned
+ * path that does not take the layer's weight types returns BREAD_ERR_QTYPE. */
 int bread_moe_forward(bread_moe_ctx_t *ctx, const bread_moe_layer_t *layer,
                       const float *d_x_normed, float *d_hidden, int n_tokens,
                       int32_t *d_idx, float *d_w, float *d_gsh, bread_stream_t stream);
