@@ -82,7 +82,6 @@ struct bread_grouped_ws {
     int *pos_of = nullptr;                // sorted position of pair (t, k) [max_tokens*K]
     void *tiles = nullptr;                // tiles of the expert GEMMs
     int *n_tiles = nullptr;               // routed tiles, and all with the shared expert's
-    float *h = nullptr;                   // SwiGLU rows by tile [tiles][32][Imax]
     float *eo = nullptr;                  // expert outputs by pair [max_tokens*(K+1)][H]
 };
 

@@ -620,7 +620,7 @@ struct GgArgs {
     const int *pair_tok;
     const MtTile *tiles;
     const int *n_tiles;
-    float *h;                  // SwiGLU rows by tile [tiles][MT][hstride]
+    float *h;                  // SwiGLU rows by pair [pairs][hstride]
     float *eo;                 // expert outputs by pair [pairs][H]
     int E, nsb, rows;          // superblocks of the contraction, rows per expert
     int hstride;
@@ -638,7 +638,7 @@ struct GgArgs {
 struct GgItems {
     const MtTile CONST_AS *tiles;
     int lo, N, per, j, i, C;
-    int tile, chunk, e, p0, nr;  // the current item
+    int chunk, e, p0, nr;  // the current item
 
     __device__ __forceinline__ GgItems(const GgArgs &a, int chunks)
     {
@@ -656,7 +656,7 @@ struct GgItems {
     {
         j += (int)gridDim.x / NXCD;
         if (j >= per || i + j >= N) return false;
-        tile = uniform(lo + (i + j) / C);
+        const int tile = uniform(lo + (i + j) / C);
         chunk = uniform((i + j) % C);
         e = uniform(tiles[tile].e);
         p0 = uniform(tiles[tile].p0);
@@ -885,8 +885,8 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
     stage_w(m0, m1, 0);
     bool first = true;
     for (int turn = 0;; turn ^= 1, first = false) {
-        const int tile = it.tile, nr = it.nr, row0 = it.chunk * GU_ROWS + 32 * w;
-        const int ex_tok = a.pair_tok[it.p0 + min(tid & (MT - 1), nr - 1)];
+        const int p0 = it.p0, nr = it.nr, row0 = it.chunk * GU_ROWS + 32 * w;
+        const int ex_tok = a.pair_tok[p0 + min(tid & (MT - 1), nr - 1)];
         const bool more = it.next();
         matrices(n0, n1);
         tokens();
@@ -930,7 +930,7 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
         const uint32_t col = (uint32_t)(((row0 + r) & ~(QK - 1)) + 8 * u + 4 * ((c >> 5) & 1) + 2 * (c & 1) + ((c >> 1) & 1));
         // rows past nr fall outside the buffer's range: every lane issues all
         // 16 stores, which the next item's first wait leaves in flight
-        const __amdgpu_buffer_rsrc_t hb = rsrc(a.h + (size_t)tile * MT * a.hstride, (uint32_t)(nr * a.hstride * 4));
+        const __amdgpu_buffer_rsrc_t hb = rsrc(a.h + (size_t)p0 * a.hstride, (uint32_t)(nr * a.hstride * 4));
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int n = 8 * (i >> 2) + 4 * g + (i & 3);
@@ -1048,7 +1048,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
     const int hn = tid >> 4, hq = tid & 15;
     float4 va[2 * NB], vb[2 * NB];
     auto load_h = [&]() __attribute__((always_inline)) {
-        const float *hr = a.h + ((size_t)it.tile * MT + min(hn, it.nr - 1)) * a.hstride + 8 * hq;
+        const float *hr = a.h + (size_t)(it.p0 + min(hn, it.nr - 1)) * a.hstride + 8 * hq;
 #pragma unroll
         for (int k = 0; k < 2 * NB; k++) {
             va[k] = vb[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1273,9 +1273,6 @@ int bread_grouped_alloc(bread_moe_ctx_t *c)
     if (e == hipSuccess) e = hipMalloc((void **)&g.pos_of, T * K * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&g.tiles, (size_t)max_tiles(s, c->max_tokens) * sizeof(MtTile));
     if (e == hipSuccess) e = hipMalloc((void **)&g.n_tiles, 2 * sizeof(int));
-    const size_t Imax = (size_t)(s.expert_inter > s.shared_inter ? s.expert_inter : s.shared_inter);
-    if (e == hipSuccess && Imax <= MAX_INTER)
-        e = hipMalloc((void **)&g.h, (size_t)max_tiles(s, c->max_tokens) * MT * Imax * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void **)&g.eo, P * H * sizeof(float));
     return e == hipSuccess ? BREAD_OK : (e == hipErrorOutOfMemory ? BREAD_ERR_NOMEM : BREAD_ERR_HIP);
 }
@@ -1290,7 +1287,6 @@ void bread_grouped_free(bread_moe_ctx_t *c)
     (void)hipFree(g.pos_of);
     (void)hipFree(g.tiles);
     (void)hipFree(g.n_tiles);
-    (void)hipFree(g.h);
     (void)hipFree(g.eo);
     g = bread_grouped_ws{};
 }
@@ -1345,7 +1341,7 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     a.pair_tok = g.pair_tok;
     a.tiles = (const MtTile *)g.tiles;
     a.n_tiles = g.n_tiles;
-    a.h = g.h;
+    a.h = c->h;
     a.eo = g.eo;
     a.E = E;
     a.hstride = Imax;

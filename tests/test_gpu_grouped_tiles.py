@@ -43,3 +43,21 @@ def test_grouped_tile_edges(H, I, Ish, T):
     got = hd.cpu().numpy()
     assert np.array_equal(got.view(np.uint32), np.repeat(got[:1], T, axis=0).view(np.uint32))
     assert rel_l2(got, ref) < 2.0 ** -11
+
+
+def test_context_memory_per_token():
+    """What a context of the benchmark's shape takes for each token: the fp32
+    residual, input and logits, activations in operand order, SwiGLU rows and
+    expert outputs of nine pairs come to 115.5 KB; 4 KB more for
+    2 MB pages over 8192 tokens."""
+    s = api.shape()
+
+    def taken(tokens):
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        ctx = B.MoeContext(s, max_tokens=tokens)
+        n = free - torch.cuda.mem_get_info()[0]
+        ctx.close()
+        return n
+
+    assert (taken(12288) - taken(4096)) / 8192 < 120 * 1024
