@@ -1,13 +1,15 @@
-"""Edges of the grouped GEMMs' tiles (moe_grouped.hip) against the CPU oracle:
-identical tokens, so every chosen expert and the shared one take T pairs, at
-counts around the 32-pair tile; hidden sizes that end inside a 512-row chunk
-of the down kernel; one superblock and two of intermediate size, the shared
-expert's equal to the routed one's (one launch) or not (two).
+"""Edges of the grouped path (moe_grouped.hip): its GEMMs' tiles, its bucketing
+and its workspace.  The tiles against the CPU oracle: identical tokens, so every
+chosen expert and the shared one take T pairs, at counts around the 32-pair
+tile; hidden sizes that end inside a 512-row chunk of the down kernel; one
+superblock and two of intermediate size, the shared expert's equal to the
+routed one's (one launch) or not (two).
 
-Bound: the Q6_K down weights are fp16 roundings of integers up to 4096, off
-by at most 1 above 2048, 2^-12 of the weight; everything else is exact or has
-22 bits.  Roundings of one row have random signs, so the relative L2 error of
-a token's output stays below twice that, 2^-11.
+Bound: the Q6_K down weights are integers up to 4096 rounded to fp16, off by 1
+where they are odd and above 2048, so by less than 2^-11 of a weight and by
+nothing below; everything else is exact or has 22 bits.  An output's products
+have random signs, as their roundings have, so errors of less than 2^-11 of
+every product leave a token's output less than 2^-11 off in relative L2.
 """
 import numpy as np
 import pytest
@@ -43,6 +45,30 @@ def test_grouped_tile_edges(H, I, Ish, T):
     got = hd.cpu().numpy()
     assert np.array_equal(got.view(np.uint32), np.repeat(got[:1], T, axis=0).view(np.uint32))
     assert rel_l2(got, ref) < 2.0 ** -11
+
+
+@pytest.mark.parametrize("T,E", [(2048, 24), (2049, 24), (2050, 1000), (4100, 12)])
+def test_bucketing_passes(T, E):
+    """16,384 pairs are what the bucketing keeps in registers; more of them take
+    a second and a third pass, here with ends inside a pass and inside its 1,024
+    threads.  A pair in the wrong place gives its token another expert's output.
+    Same bound as above."""
+    s = api.shape(hidden=256, expert_inter=256, shared_inter=256, n_experts=E, top_k=8)
+    t = api.synth_layer_tensors(s, seed=9, layer=0)
+    x = torch.randn(T, 256, device=DEV, generator=torch.Generator(device=DEV).manual_seed(T))
+    out = []
+    for path in (api.PATH_GROUPED, api.PATH_PER_TOKEN):
+        ctx = B.MoeContext(s, max_tokens=T)
+        ctx.set_path(path)
+        hd = torch.zeros(T, 256, device=DEV)
+        idx, w, _ = ctx.forward(t.desc(), x, hd, T, want_routing=True)
+        torch.cuda.synchronize()
+        assert ctx.check_device() == 0
+        out.append([v.cpu().numpy() for v in (hd, idx, w)])
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    err = np.linalg.norm(out[0][0] - out[1][0], axis=1) / np.linalg.norm(out[1][0], axis=1)
+    assert err.max() < 2.0 ** -11
 
 
 def test_context_memory_per_token():
