@@ -336,7 +336,7 @@ __global__ __launch_bounds__(256) void k_gateup(bread_moe_layer_t L, const float
 // One wave per (token, output row): down rows of every slot, combined in the
 // reference order (one_layer.cu:1447-1469): the shared expert (when
 // `shared`), then the routed experts by rank.
-// Latency bound: 16 MB of weights over 2048 waves a token.  A superblock is
+// Latency bound: 6.9 MB of weights over 2048 waves a token.  A superblock is
 // eight lanes' work, so a row of 512 columns would leave 48 of 64 lanes idle,
 // and the slots one after another wait for memory each; the wave takes eight
 // (slot, superblock) pairs at once instead, two passes in flight, and sums

@@ -21,8 +21,10 @@
 // run in fp32 at fewer tokens, carry that rest in a second operand and scale
 // the lo terms (LO_EXP): their inputs are off by 2^-23 at most, and with exact
 // products the sums come out as near to 64-bit arithmetic as the per-token
-// kernels' (27 tokens of hidden 2048, all Q4_K: 5.5e-7 both, all Q6_K: 2.6e-7
+// kernels' (27 tokens of hidden 2048, all Q4_K: 5.5e-7 both, all Q6_K: 2.5e-7
 // both).
+// A row that holds an infinity has NaN terms, so where fp32 sums would give
+// some outputs of that token as infinities they are NaN.
 //
 // Kernels per layer, stream-ordered:
 //   k_route_seq   router logits in the reference's sequential order
@@ -34,16 +36,13 @@
 //                 operand order, sub-block sums, shared-gate logit
 //   k_mt_bucket   one workgroup: expert histogram, token lists by expert,
 //                 tiles of 32 pairs
-//   k_gateup      per (tile, 128 rows): gate and up GEMMs and SwiGLU
+//   k_gateup_gg   per (tile, 128 rows): gate and up GEMMs and SwiGLU
 //   k_down_gg     per (tile, 512 rows): the tile's SwiGLU rows split into hi/lo
 //                 fp16 with a row scale, then the down GEMM
 //   k_mt_combine  per token: shared expert, then routed experts in rank order
 // The shared expert is expert index E with every token, so both GEMMs treat
 // it like a routed expert with its own weights.
 #include <float.h>
-#include <stdlib.h>
-
-#include <type_traits>
 
 #include "bread_internal.h"
 #include "bread_device.h"
@@ -468,9 +467,11 @@ __device__ __forceinline__ uint4 lo_operand(const uint4 &w)
 
 // Operand maker of one unit (32 weight rows of one superblock): constants
 // from the superblock's header, then a step's eight weights; the scaling of
-// the sums.  prepare() sets bad when the superblock is outside the range that
-// fp16 weights can hold (checked where `flag`): Q4_K |d| >= 64 or |dmin| >=
-// 1024, Q6_K |d sc| >= 2047, or NaN.
+// the sums.  prepare() sets bad (where `flag`, the layers of the reference GPU
+// path's types) for Q4_K |d| >= 64 or |dmin| >= 1024, Q6_K |d sc| >= 2047, or
+// NaN: superblocks whose weights fp16 does not hold.  The operands here are
+// integers, so finite ones come out right all the same; the flag stays because
+// callers know such layers by it (BREAD_DEV_ERR_RANGE).
 template <int QT, bool X>
 struct Unit;
 
@@ -723,11 +724,14 @@ struct XRead {
 // Everything comes by direct-to-LDS loads whose adjacent lanes read adjacent
 // memory: a load whose lanes are 64 rows costs the address unit a cycle a
 // lane, and with the weights loaded so (16 bytes of a row a lane) issuing a
-// superblock's loads took 2,500-5,000 cycles of an iteration of 8,500.  Weights: a wave's 2 x 32 rows of a superblock (9 KB) into a buffer
-// of its own, moved to registers when the superblock begins, which frees the
-// buffer for the next one.  Activations: half a superblock of the tile's 32
-// rows (16 KB) into one of two buffers, a half ahead.  A barrier each half;
-// 70 KB of LDS, two workgroups a CU.
+// superblock's loads took 2,500-5,000 cycles of an iteration of 8,500.
+// Weights: a wave's 2 x 32 rows of a superblock (9 KB) into a buffer of its
+// own, moved to registers when the superblock begins, which frees the buffer
+// for the next one.  Activations: half a superblock of the tile's 32 rows (16
+// KB) into one of two buffers, a half ahead.  A barrier each half; 73 KB of
+// LDS, two workgroups a CU, so 256 vector registers a wave: 207 in use, 216
+// (Q4_K) to 245 (Q6_K) with X.  21-29 scalar registers spill into vector ones
+// in the Q4_K forms, outside the steps.
 // Q6_K gate or up (no reference GPU layout) loads its weights straight into
 // registers: its 210-byte superblocks are 2-byte aligned.
 //
@@ -746,14 +750,14 @@ constexpr int W_BUF = W_LOADS * WAVE;  // the last load's idle lanes repeat the 
 
 // X: the exact operands of layers of other types than the reference GPU path's
 template <int Q0, int Q1, bool X>
-__global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
+__global__ __launch_bounds__(GG_THREADS, 2) void k_gateup_gg(const GgArgs a)
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K;
     constexpr bool X0 = Q0 != Q4, X1 = Q1 != Q4, SUMS = Q0 == Q4 || Q1 == Q4;
     // a variable for each buffer: a read of one that a direct-to-LDS load may
     // write waits for all such loads
     __shared__ uint4 sA0[MT][32], sA1[MT][32], sS[MT][2];
-    __shared__ uint4 sW[GG_WAVES][(Q0 == Q4) + (Q1 == Q4) ? (Q0 == Q4) + (Q1 == Q4) : 1][W_BUF];
+    __shared__ uint4 sW[GG_WAVES][Q0 == Q4 && Q1 == Q4 ? 2 : 1][W_BUF];
     __shared__ int sexp[2][MT];
     const int tid = (int)threadIdx.x, w = wave_id(), lane = lane_id();
     const int g = lane >> 5, r = lane & 31;
@@ -927,7 +931,8 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
         // unit's place (unit_base), for k_down_gg's loads
         const int c = (row0 + r) & (QK - 1);
         const int u = 2 * (8 * ((c >> 6) & 1) + ((c >> 2) & 7)) + (c >> 7);
-        const uint32_t col = (uint32_t)(((row0 + r) & ~(QK - 1)) + 8 * u + 4 * ((c >> 5) & 1) + 2 * (c & 1) + ((c >> 1) & 1));
+        const uint32_t col =
+            (uint32_t)(((row0 + r) & ~(QK - 1)) + 8 * u + 4 * ((c >> 5) & 1) + 2 * (c & 1) + ((c >> 1) & 1));
         // rows past nr fall outside the buffer's range: every lane issues all
         // 16 stores, which the next item's first wait leaves in flight
         const __amdgpu_buffer_rsrc_t hb = rsrc(a.h + (size_t)p0 * a.hstride, (uint32_t)(nr * a.hstride * 4));
@@ -935,8 +940,9 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup(const GgArgs a)
         for (int i = 0; i < 16; i++) {
             const int n = 8 * (i >> 2) + 4 * g + (i & 3);
             const int ex = sexp[turn][n];
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, silu_mul(ldexpf(t0[i], ex), ldexpf(t1[i], ex))),
-                                                  hb, 4 * (uint32_t)(n * a.hstride) + 4 * col, 0, 0);
+            const float v = silu_mul(ldexpf(t0[i], ex), ldexpf(t1[i], ex));
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), hb,
+                                                  4 * (uint32_t)(n * a.hstride) + 4 * col, 0, 0);
         }
         if (!more) break;
         m0 = n0;
@@ -1002,7 +1008,7 @@ __device__ __forceinline__ void take_unit(Raw<BREAD_QTYPE_Q6_K> &R, const uint4 
     R.d = p[52] >> (8 * sh);
 }
 
-// X as in k_gateup
+// X as in k_gateup_gg
 template <int QT, bool X>
 __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
 {
@@ -1236,11 +1242,11 @@ void launch_gateup(const GgArgs &a, int tg, int tu, bool exact, int tiles, int c
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K, Q6 = BREAD_QTYPE_Q6_K;
     const dim3 grid = gg_grid(tiles, a.rows / GU_ROWS, 2 * cus), block(GG_THREADS);
-    if (!exact) hipLaunchKernelGGL((k_gateup<Q4, Q4, false>), grid, block, 0, st, a);
-    else if (tg == Q4 && tu == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q4, true>), grid, block, 0, st, a);
-    else if (tg == Q4) hipLaunchKernelGGL((k_gateup<Q4, Q6, true>), grid, block, 0, st, a);
-    else if (tu == Q4) hipLaunchKernelGGL((k_gateup<Q6, Q4, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_gateup<Q6, Q6, true>), grid, block, 0, st, a);
+    if (!exact) hipLaunchKernelGGL((k_gateup_gg<Q4, Q4, false>), grid, block, 0, st, a);
+    else if (tg == Q4 && tu == Q4) hipLaunchKernelGGL((k_gateup_gg<Q4, Q4, true>), grid, block, 0, st, a);
+    else if (tg == Q4) hipLaunchKernelGGL((k_gateup_gg<Q4, Q6, true>), grid, block, 0, st, a);
+    else if (tu == Q4) hipLaunchKernelGGL((k_gateup_gg<Q6, Q4, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_gateup_gg<Q6, Q6, true>), grid, block, 0, st, a);
 }
 
 void launch_down(const GgArgs &a, int td, bool exact, int tiles, int cus, hipStream_t st)
