@@ -340,7 +340,12 @@ __global__ __launch_bounds__(256) void k_gateup(bread_moe_layer_t L, const float
 // eight lanes' work, so a row of 512 columns would leave 48 of 64 lanes idle,
 // and the slots one after another wait for memory each; the wave takes eight
 // (slot, superblock) pairs at once instead, two passes in flight, and sums
-// them in slot order.  One token, 8 slots of 512: 15.4 -> 7.2 us on MI355X.
+// them in slot order.  One token, 8 slots of 512: 15.4 -> 7.2 us on MI355X.  A
+// single slot (top 1) leaves nothing to fill the lanes with and takes the row's
+// own loop, which has less to do: hidden 2048, one slot of 256 in Q4_K, 40
+// tokens: a layer in 152 us as pairs, 103 so.  (A kernel of its own: the two
+// in one take registers that cost the pairs 5 % at 40 tokens.)
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_down(bread_moe_layer_t L, const int32_t *__restrict__ idx,
                                               const float *__restrict__ w, const float *__restrict__ gsh,
                                               const float *__restrict__ h, float *__restrict__ hidden, int H,
@@ -360,6 +365,14 @@ __global__ __launch_bounds__(256) void k_down(bread_moe_layer_t L, const int32_t
         const float sh = wave_sum(kq_row_partial(
             st, (const uint8_t *)L.down_shexp + (uint64_t)r * bread_expert_row_bytes(st, Ish), Ish / QK, ht, lane));
         acc += sigmoidf_ref(gsh[t]) * sh;
+    }
+    if constexpr (ONE) {
+        const uint64_t rb = bread_expert_row_bytes(dt, I);
+        const int e = checked_expert(idx[t], E, err);
+        const uint8_t *d = (const uint8_t *)L.down_exps + (uint64_t)e * L.down_expert_bytes + r * rb;
+        acc += w[t] * wave_sum(kq_row_partial(dt, d, I / QK, ht + Imax, lane));
+        if (lane == 0) hidden[(size_t)t * H + r] = acc;
+        return;
     }
     const int nb = I / QK, np = K * nb;
     const uint32_t bb = (uint32_t)bread_expert_row_bytes(dt, QK);
@@ -514,6 +527,16 @@ __global__ __launch_bounds__(256) void k_f16_out(const float *__restrict__ h32, 
 // Launchers
 // ---------------------------------------------------------------------------
 
+static void launch_down(const bread_moe_ctx_t *c, const bread_moe_layer_t *L, const int32_t *idx, const float *w,
+                        float *hidden, int T, int shared, hipStream_t st)
+{
+    const bread_moe_shape_t &s = c->shape;
+    const dim3 grid((unsigned)(((uint64_t)T * s.hidden + 3) / 4));
+    hipLaunchKernelGGL(s.top_k == 1 ? k_down<true> : k_down<false>, grid, dim3(256), 0, st, *L, idx, w, c->gsh, c->h,
+                       hidden, s.hidden, s.expert_inter, s.shared_inter, s.top_k, T, s.n_experts, shared,
+                       &c->dsync->error.v);
+}
+
 int bread_launch_moe_multi(bread_moe_ctx_t *c, const bread_moe_layer_t *L, const float *x, float *hidden, int T,
                            hipStream_t st)
 {
@@ -525,10 +548,7 @@ int bread_launch_moe_multi(bread_moe_ctx_t *c, const bread_moe_layer_t *L, const
     hipLaunchKernelGGL(k_gateup, dim3((unsigned)((gu_waves + 3) / 4)), dim3(256), 0, st, *L, x, c->idx, c->h,
                        s.hidden, s.expert_inter, s.shared_inter, s.top_k, T, s.n_experts, 1, &c->dsync->error.v);
     BREAD_HIP(hipGetLastError());
-    const uint64_t dn_waves = (uint64_t)T * s.hidden;
-    hipLaunchKernelGGL(k_down, dim3((unsigned)((dn_waves + 3) / 4)), dim3(256), 0, st, *L, c->idx, c->w, c->gsh,
-                       c->h, hidden, s.hidden, s.expert_inter, s.shared_inter, s.top_k, T, s.n_experts, 1,
-                       &c->dsync->error.v);
+    launch_down(c, L, c->idx, c->w, hidden, T, 1, st);
     BREAD_HIP(hipGetLastError());
     return BREAD_OK;
 }
@@ -697,10 +717,7 @@ extern "C" int bread_moe_expert_block(bread_moe_ctx_t *c, const bread_moe_layer_
     hipLaunchKernelGGL(k_gateup, dim3((unsigned)((gu_waves + 3) / 4)), dim3(256), 0, st, *L, x, idx, c->h,
                        s.hidden, s.expert_inter, s.shared_inter, s.top_k, T, s.n_experts, 0, &c->dsync->error.v);
     BREAD_HIP(hipGetLastError());
-    const uint64_t dn_waves = (uint64_t)T * s.hidden;
-    hipLaunchKernelGGL(k_down, dim3((unsigned)((dn_waves + 3) / 4)), dim3(256), 0, st, *L, idx, w, c->gsh, c->h,
-                       hidden, s.hidden, s.expert_inter, s.shared_inter, s.top_k, T, s.n_experts, 0,
-                       &c->dsync->error.v);
+    launch_down(c, L, idx, w, hidden, T, 0, st);
     BREAD_HIP(hipGetLastError());
     return BREAD_OK;
 }

@@ -16,7 +16,7 @@ import breadv2_amd as B
 from breadv2_amd import api
 from oracle import oracle as O
 
-from helpers import assert_moe_close, host_layer
+from helpers import assert_moe_close, host_layer, rel_l2
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -95,6 +95,27 @@ def test_mixed_type_layer():
     ref = hidden.copy()
     O.expert_block(hl, x, ref, idx, w)
     assert_moe_close(got, ref)
+
+
+@pytest.mark.parametrize("K,I", [(1, 256), (1, 512), (1, 2304), (2, 256), (3, 768), (4, 1024), (5, 1536)])
+@pytest.mark.parametrize("down", [api.QTYPE_Q4_K, api.QTYPE_Q6_K])
+def test_slots_and_superblocks(K, I, down):
+    """One slot, and (slot, superblock) pairs that fill a pass of eight or two
+    of them, end inside one, or put a slot's superblocks in two.  Sums of up to
+    2304 products in fp32 on either side, 2^-24 each with random signs: 3e-6."""
+    s = api.shape(hidden=256, expert_inter=I, shared_inter=256, n_experts=6, top_k=K)
+    types = (api.QTYPE_Q4_K, api.QTYPE_Q4_K, down, api.QTYPE_Q4_K, api.QTYPE_Q4_K, api.QTYPE_Q6_K)
+    t = api.synth_layer_tensors(s, seed=779, layer=0, types=types)
+    torch.cuda.synchronize()
+    T, rng = 3, np.random.default_rng(K * I)
+    x = rng.standard_normal((T, s.hidden)).astype(np.float32)
+    idx = np.stack([rng.permutation(6)[:K] for _ in range(T)]).astype(np.int32)
+    w = rng.uniform(-1, 1, (T, K)).astype(np.float32)
+    hidden = np.zeros((T, s.hidden), np.float32)
+    got = run(s, t, x, hidden, idx, w)
+    ref = hidden.copy()
+    O.expert_block(host_layer(t), x, ref, idx, w)
+    assert rel_l2(got, ref) < 1e-5
 
 
 def test_out_of_range_index_is_flagged(layer):
