@@ -624,31 +624,36 @@ struct GgArgs {
     const int *n_tiles;
     float *h;                  // SwiGLU rows by pair [pairs][hstride]
     float *eo;                 // expert outputs by pair [pairs][H]
-    int E, nsb, rows;          // superblocks of the contraction, rows per expert
+    int E;
+    int nsb, nsb_sh;           // superblocks of the contraction: routed, shared
+    int rows, rows_sh;         // rows of an expert
     int hstride;
-    int sel;                   // 0: all tiles, 1: routed, 2: shared
+    int sel;                   // 1: the routed tiles, 2: the shared ones, 3: both
     int flag;                  // report superblocks outside the fp16 range
 };
 
 #define CONST_AS __attribute__((address_space(4)))  // read by scalar loads
 
 // The items of a workgroup: (tile, chunk of rows), the chunks of a tile in
-// sequence, C a tile.  Workgroups go to the 8 XCDs round-robin by linear id and
+// sequence, C a tile (C_sh of the shared expert's, which come last and may have
+// another size).  Workgroups go to the 8 XCDs round-robin by linear id and
 // each XCD has its own L2, so XCD L % 8 takes a contiguous eighth, where a
 // tile's chunks share its activations and an expert's tiles its weights; its
 // workgroups take turns.
 struct GgItems {
     const MtTile CONST_AS *tiles;
-    int lo, N, per, j, i, C;
+    int routed, first_sh, N, per, j, i, C, C_sh;
     int chunk, e, p0, nr;  // the current item
 
-    __device__ __forceinline__ GgItems(const GgArgs &a, int chunks)
+    __device__ __forceinline__ GgItems(const GgArgs &a, int chunks, int chunks_sh)
     {
         const int CONST_AS *n = (const int CONST_AS *)a.n_tiles;
         tiles = (const MtTile CONST_AS *)a.tiles;
         C = chunks;
-        lo = a.sel == 2 ? n[0] : 0;
-        N = ((a.sel == 1 ? n[0] : n[1]) - lo) * C;
+        C_sh = chunks_sh;
+        first_sh = n[0];
+        routed = a.sel & 1 ? n[0] * C : 0;
+        N = routed + (a.sel & 2 ? (n[1] - n[0]) * C_sh : 0);
         per = (N + NXCD - 1) / NXCD;
         j = (int)blockIdx.x / NXCD - (int)gridDim.x / NXCD;
         i = ((int)blockIdx.x % NXCD) * per;
@@ -658,8 +663,10 @@ struct GgItems {
     {
         j += (int)gridDim.x / NXCD;
         if (j >= per || i + j >= N) return false;
-        const int tile = uniform(lo + (i + j) / C);
-        chunk = uniform((i + j) % C);
+        const bool sh = i + j >= routed;
+        const int k = i + j - (sh ? routed : 0), c = sh ? C_sh : C;
+        const int tile = uniform((sh ? first_sh : 0) + k / c);
+        chunk = uniform(k % c);
         e = uniform(tiles[tile].e);
         p0 = uniform(tiles[tile].p0);
         nr = uniform(tiles[tile].nr);
@@ -731,7 +738,7 @@ struct XRead {
 // for the next one.  Activations: half a superblock of the tile's 32 rows (16
 // KB) into one of two buffers, a half ahead.  A barrier each half; 73 KB of
 // LDS, two workgroups a CU, so 256 vector registers a wave: 207 in use, 208
-// (Q4_K) to 245 (Q6_K) with X.  21-29 scalar registers spill into vector ones
+// (Q4_K) to 245 (Q6_K) with X.  19-29 scalar registers spill into vector ones
 // in the Q4_K forms, outside the steps.
 // Q6_K gate or up (no reference GPU layout) loads its weights straight into
 // registers: its 210-byte superblocks are 2-byte aligned.
@@ -762,7 +769,7 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup_gg(const GgArgs a)
     __shared__ int sexp[2][MT];
     const int tid = (int)threadIdx.x, w = wave_id(), lane = lane_id();
     const int g = lane >> 5, r = lane & 31;
-    GgItems it(a, a.rows / GU_ROWS);
+    GgItems it(a, a.rows / GU_ROWS, a.rows_sh / GU_ROWS);
     if (!it.next()) return;
     const uint32_t rb0 = (uint32_t)a.nsb * Raw<Q0>::BYTES, rb1 = (uint32_t)a.nsb * Raw<Q1>::BYTES;
     // the item's matrices, from the wave's first row (n0, n1: the next item's)
@@ -1023,10 +1030,11 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
     __shared__ int sexp[MT];
     const int tid = (int)threadIdx.x, w = wave_id(), lane = lane_id();
     const int g = lane >> 5, r = lane & 31;
-    GgItems it(a, (a.rows + DN_ROWS - 1) / DN_ROWS);
+    const int chunks = (a.rows + DN_ROWS - 1) / DN_ROWS;
+    GgItems it(a, chunks, chunks);
     if (!it.next()) return;
-    const int nb = a.nsb;
-    const uint32_t rb = (uint32_t)nb * Raw<QT>::BYTES;
+    // superblocks of `it`'s rows
+    auto superblocks = [&]() __attribute__((always_inline)) { return it.e == a.E ? a.nsb_sh : a.nsb; };
     // the item's matrix from the wave's first row; blocks past the end
     // repeat the last one and are not stored
     auto matrix = [&]() __attribute__((always_inline)) {
@@ -1035,26 +1043,28 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
     auto block_row = [&](int chunk, int blk) __attribute__((always_inline)) {
         return chunk * DN_ROWS + 32 * (DN_BLOCKS * w + blk);
     };
-    // piece 64 j + lane of a unit: its row's offset and the piece's
+    // piece 64 j + lane of a unit: its row and the piece's offset
     uint32_t ro[UNIT_LD<QT>], po[UNIT_LD<QT>];
 #pragma unroll
     for (int j = 0; j < UNIT_LD<QT>; j++) {
         const uint32_t c = (uint32_t)min(64 * j + lane, 32 * ROW_CH<QT> - 1);
-        ro[j] = c / ROW_CH<QT> * rb;
+        ro[j] = c / ROW_CH<QT>;
         po[j] = 16 * min(c % ROW_CH<QT>, (uint32_t)(QT == Q4 ? 8 : 13));
     }
     // unit u: block u / nb, superblock u % nb
-    auto stage_w = [&](const uint8_t *m, int chunk, int u) __attribute__((always_inline)) {
+    auto stage_w = [&](const uint8_t *m, int chunk, int nb, int u) __attribute__((always_inline)) {
         const int blk = nb == 2 ? u >> 1 : u, b = u - blk * nb;
+        const uint32_t rb = (uint32_t)nb * Raw<QT>::BYTES;
         const uint8_t *p = m + (uint64_t)(uint32_t)min(block_row(chunk, blk), a.rows - 32) * rb;
 #pragma unroll
         for (int j = 0; j < UNIT_LD<QT>; j++)
-            lds_load16(p + (((ro[j] + (uint32_t)b * Raw<QT>::BYTES) & ~15u) + po[j]), &sW[w][64 * j]);
+            lds_load16(p + (((ro[j] * rb + (uint32_t)b * Raw<QT>::BYTES) & ~15u) + po[j]), &sW[w][64 * j]);
     };
     // 16 threads a token, each the units q + 16 k of its superblocks
     const int hn = tid >> 4, hq = tid & 15;
     float4 va[2 * NB], vb[2 * NB];
     auto load_h = [&]() __attribute__((always_inline)) {
+        const int nb = superblocks();
         const float *hr = a.h + (size_t)(it.p0 + min(hn, it.nr - 1)) * a.hstride + 8 * hq;
 #pragma unroll
         for (int k = 0; k < 2 * NB; k++) {
@@ -1065,7 +1075,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
             }
         }
     };
-    auto split_h = [&]() __attribute__((always_inline)) {
+    auto split_h = [&](int nb) __attribute__((always_inline)) {
         float mx = 0.f;
 #pragma unroll
         for (int k = 0; k < 2 * NB; k++) {
@@ -1113,11 +1123,12 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
     const uint8_t *m = matrix();
     bool stores = false;  // the last unit stored
     load_h();
-    stage_w(m, it.chunk, 0);
+    stage_w(m, it.chunk, superblocks(), 0);
     for (;;) {
-        const int chunk = it.chunk, p0 = it.p0, nr = it.nr;
+        const int chunk = it.chunk, p0 = it.p0, nr = it.nr, nb = superblocks();
+        const uint32_t rb = (uint32_t)nb * Raw<QT>::BYTES;
         const uint8_t *mc = m;
-        split_h();
+        split_h(nb);
         gg_bar();
         const bool more = it.next();
         m = matrix();
@@ -1131,7 +1142,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
             __builtin_amdgcn_sched_barrier(0);
             const bool last = u + 1 == DN_BLOCKS * nb;
             if (last) load_h();
-            stage_w(last ? m : mc, last ? it.chunk : chunk, last ? 0 : u + 1);
+            stage_w(last ? m : mc, last ? it.chunk : chunk, last ? superblocks() : nb, last ? 0 : u + 1);
             __builtin_amdgcn_sched_barrier(0);
             U.prepare(R, C, g, a.flag != 0 && row0 < a.rows, bad);
             f32x16 c0 = zero16(), c1 = zero16();
@@ -1242,7 +1253,7 @@ dim3 gg_grid(int tiles, int C, int resident)
 void launch_gateup(const GgArgs &a, int tg, int tu, bool exact, int tiles, int cus, hipStream_t st)
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K, Q6 = BREAD_QTYPE_Q6_K;
-    const dim3 grid = gg_grid(tiles, a.rows / GU_ROWS, 2 * cus), block(GG_THREADS);
+    const dim3 grid = gg_grid(tiles, max(a.rows, a.rows_sh) / GU_ROWS, 2 * cus), block(GG_THREADS);
     if (!exact) hipLaunchKernelGGL((k_gateup_gg<Q4, Q4, false>), grid, block, 0, st, a);
     else if (tg == Q4 && tu == Q4) hipLaunchKernelGGL((k_gateup_gg<Q4, Q4, true>), grid, block, 0, st, a);
     else if (tg == Q4) hipLaunchKernelGGL((k_gateup_gg<Q4, Q6, true>), grid, block, 0, st, a);
@@ -1353,24 +1364,23 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     a.E = E;
     a.hstride = Imax;
     a.flag = standard ? 1 : 0;
-    // one launch takes tiles of one geometry and type: the shared expert's
-    // ride along with the routed ones' where both agree
-    const bool one_gu = s.expert_inter == s.shared_inter && L->gate_type == L->gate_shexp_type &&
-                        L->up_type == L->up_shexp_type;
-    const bool one_dn = s.expert_inter == s.shared_inter && L->down_type == L->down_shexp_type;
+    // one launch takes tiles of one type: the shared expert's ride along with
+    // the routed ones' where they agree
+    const bool one_gu = L->gate_type == L->gate_shexp_type && L->up_type == L->up_shexp_type;
+    const bool one_dn = L->down_type == L->down_shexp_type;
     a.w0 = (const uint8_t *)L->gate_exps;
     a.w1 = (const uint8_t *)L->up_exps;
     a.st0 = L->gate_expert_bytes;
     a.st1 = L->up_expert_bytes;
     a.sw0 = (const uint8_t *)L->gate_shexp;
     a.sw1 = (const uint8_t *)L->up_shexp;
-    a.nsb = H / QK;
+    a.nsb = a.nsb_sh = H / QK;
     a.rows = s.expert_inter;
-    a.sel = one_gu ? 0 : 1;
+    a.rows_sh = s.shared_inter;
+    a.sel = one_gu ? 3 : 1;
     launch_gateup(a, L->gate_type, L->up_type, !standard, tiles, g.cus, st);
     BREAD_HIP(hipGetLastError());
     if (!one_gu) {
-        a.rows = s.shared_inter;
         a.sel = 2;
         launch_gateup(a, L->gate_shexp_type, L->up_shexp_type, !standard, tiles, g.cus, st);
         BREAD_HIP(hipGetLastError());
@@ -1379,12 +1389,12 @@ int bread_launch_moe_grouped(bread_moe_ctx_t *c, const bread_moe_layer_t *L, con
     a.st0 = a.st1 = L->down_expert_bytes;
     a.sw0 = a.sw1 = (const uint8_t *)L->down_shexp;
     a.nsb = s.expert_inter / QK;
-    a.rows = H;
-    a.sel = one_dn ? 0 : 1;
+    a.nsb_sh = s.shared_inter / QK;
+    a.rows = a.rows_sh = H;
+    a.sel = one_dn ? 3 : 1;
     launch_down(a, L->down_type, !standard, tiles, g.cus, st);
     BREAD_HIP(hipGetLastError());
     if (!one_dn) {
-        a.nsb = s.shared_inter / QK;
         a.sel = 2;
         launch_down(a, L->down_shexp_type, !standard, tiles, g.cus, st);
         BREAD_HIP(hipGetLastError());
