@@ -626,30 +626,28 @@ extern "C" int bread_stack_loop_tokens(void)
 // an expert's rows once for every token that chose it, so their time grows by
 // the R = K I + Ish rows a token has; the grouped path's is flat for few tokens,
 // at its router, its launches and one tile's chain.  They meet at some number of
-// tokens T that the types set and, for smaller layers, at some T R (twice that
-// where the shared expert has a size of its own, hence launches of its own).
-// us a layer on MI355X, uniform routing, per-token / grouped:
-//   H, I, Ish, E, K           all Q4_K               Q6_K routed down          all Q6_K
-//   2048, 512, 512, 256, 8    6: 75 / 72             14: 128 / 129             16: 177 / 176
-//                             16: 144 / 106          20: 180 / 139             32: 327 / 244
-//   2048, 512, 512, 256, 2    8: 63 / 66, 10: 70 / 66    14: 86 / 86           16: 99 / 105, 20: 118 / 107
-//   1024, 512, 512, 64, 8     6: 53 / 51             12: 81 / 71               16: 117 / 75
-//   1024, 256, 512, 32, 4     16: 66 / 70, 20: 75 / 70   20: 73 / 74           24: 93 / 109, 32: 117 / 110
-//   768, 256, 512, 24, 4      16: 58 / 64, 20: 67 / 64   20: 66 / 68           24: 83 / 101, 32: 101 / 101
-//   512, 256, 256, 24, 4      10: 33 / 35, 12: 38 / 36   16: 44 / 47, 20: 49 / 47    16: 47 / 46
-//   256, 256, 256, 8, 2       16: 29 / 31, 20: 32 / 31   24: 37 / 43, 32: 44 / 42    20: 36 / 39, 24: 41 / 39
-//   4096, 512, 512, 128, 8    6: 119 / 118           12: 208 / 203             16: 342 / 316
+// tokens T that the types set and, for smaller layers, at some T R.  us a layer on
+// MI355X, uniform routing, per-token / grouped, on either side of the line:
+//   H, I, Ish, E, K           all Q4_K              Q6_K shared down       all Q6_K
+//   2048, 512, 512, 256, 8    5: 64/71  6: 72/72    13: 120/117 14: 127/118   15: 162/169 16: 176/171
+//   2048, 512, 512, 64, 8     5: 62/69  6: 70/68    13: 118/91  14: 124/92    15: 147/110 16: 155/110
+//   2048, 512, 512, 256, 2    9: 66/65 10: 69/65    15: 91/87   16: 96/86     18: 108/106 20: 117/106
+//   1024, 512, 512, 64, 8     5: 45/50  6: 53/51    13: 86/72   14: 91/72     15: 109/75  16: 117/76
+//   1024, 256, 512, 32, 4     9: 46/47 10: 48/48    15: 63/63   16: 66/63     18: 76/68   20: 79/68
+//   768, 256, 512, 24, 4      9: 42/44 10: 44/44    15: 56/59   16: 58/59     18: 67/64   20: 72/64
+//   512, 256, 256, 24, 4     11: 37/36 12: 39/36    18: 48/48   20: 50/48     22: 60/47   24: 64/47
+//   2048, 256, 256, 64, 4    11: 72/60 12: 75/60    18: 101/73  20: 109/73    22: 122/98  24: 131/98
+//   256, 256, 256, 8, 2      18: 31/31 20: 32/31    28: 42/43   32: 45/43     (32: 49/39)
+//   4096, 512, 512, 128, 8    5: 104/114 6: 117/114 13: 218/181 14: 233/185   15: 319/308 16: 339/311
 // (Q6_K gate and up weights are gathered a row a lane.)
 static bool grouped_takes_mix(const bread_moe_shape_t &s, const bread_moe_layer_t *L, int T, const float *hidden)
 {
     const int Q4 = BREAD_QTYPE_Q4_K;
     const bool gu_q4 = L->gate_type == Q4 && L->up_type == Q4 && L->gate_shexp_type == Q4 && L->up_shexp_type == Q4;
     const bool dn_q4 = L->down_type == Q4 && L->down_shexp_type == Q4;
-    const bool one_size = s.expert_inter == s.shared_inter;
     const int64_t rows = (int64_t)T * ((int64_t)s.top_k * s.expert_inter + s.shared_inter);
-    const int tokens = !gu_q4 ? 16 : dn_q4 ? 6 : 14;
-    const int least = !gu_q4 ? (one_size ? 30000 : 49000) : dn_q4 ? (one_size ? 15000 : 30000) : one_size ? 22000 : 33000;
-    return T >= tokens && rows >= least && ((uintptr_t)hidden & 15) == 0;
+    return T >= (!gu_q4 ? 16 : dn_q4 ? 6 : 14) && rows >= (!gu_q4 ? 29000 : dn_q4 ? 15000 : 24000) &&
+           ((uintptr_t)hidden & 15) == 0;
 }
 
 extern "C" int bread_moe_forward(bread_moe_ctx_t *c, const bread_moe_layer_t *L, const float *x, float *hidden,

@@ -32,8 +32,8 @@ def first_grouped(mix, shape):
     """Tokens from which the grouped path takes a layer."""
     _, I, Ish, _, K = shape
     gu_q4, dn_q4 = {mix[0], mix[1], mix[3], mix[4]} == {Q4}, {mix[2], mix[5]} == {Q4}
-    tokens, same, other = (6, 15000, 30000) if gu_q4 and dn_q4 else (14, 22000, 33000) if gu_q4 else (16, 30000, 49000)
-    return max(tokens, -(-(same if I == Ish else other) // (K * I + Ish)))
+    tokens, rows = (6, 15000) if gu_q4 and dn_q4 else (14, 24000) if gu_q4 else (16, 29000)
+    return max(tokens, -(-rows // (K * I + Ish)))
 
 
 def run(s, d, x, hidden, path):
