@@ -738,7 +738,7 @@ struct XRead {
 // for the next one.  Activations: half a superblock of the tile's 32 rows (16
 // KB) into one of two buffers, a half ahead.  A barrier each half; 73 KB of
 // LDS, two workgroups a CU, so 256 vector registers a wave: 207 in use, 208
-// (Q4_K) to 245 (Q6_K) with X.  19-29 scalar registers spill into vector ones
+// (Q4_K) to 245 (Q6_K) with X.  20-30 scalar registers spill into vector ones
 // in the Q4_K forms, outside the steps.
 // Q6_K gate or up (no reference GPU layout) loads its weights straight into
 // registers: its 210-byte superblocks are 2-byte aligned.
@@ -898,6 +898,7 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup_gg(const GgArgs a)
     bool first = true;
     for (int turn = 0;; turn ^= 1, first = false) {
         const int p0 = it.p0, nr = it.nr, row0 = it.chunk * GU_ROWS + 32 * w;
+        float *hp = uniform_ptr(a.h + (size_t)p0 * a.hstride);
         const int ex_tok = a.pair_tok[p0 + min(tid & (MT - 1), nr - 1)];
         const bool more = it.next();
         matrices(n0, n1);
@@ -943,7 +944,7 @@ __global__ __launch_bounds__(GG_THREADS, 2) void k_gateup_gg(const GgArgs a)
             (uint32_t)(((row0 + r) & ~(QK - 1)) + 8 * u + 4 * ((c >> 5) & 1) + 2 * (c & 1) + ((c >> 1) & 1));
         // rows past nr fall outside the buffer's range: every lane issues all
         // 16 stores, which the next item's first wait leaves in flight
-        const __amdgpu_buffer_rsrc_t hb = rsrc(a.h + (size_t)p0 * a.hstride, (uint32_t)(nr * a.hstride * 4));
+        const __amdgpu_buffer_rsrc_t hb = rsrc(hp, (uint32_t)(nr * a.hstride * 4));
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int n = 8 * (i >> 2) + 4 * g + (i & 3);
@@ -1016,8 +1017,10 @@ __device__ __forceinline__ void take_unit(Raw<BREAD_QTYPE_Q6_K> &R, const uint4 
     R.d = p[52] >> (8 * sh);
 }
 
-// X as in k_gateup_gg
-template <int QT, bool X>
+// X as in k_gateup_gg.  TWO: the shared expert's intermediate size is not the
+// routed ones' (the superblocks of an item's rows then come with the item, 0.3
+// us of 20 where all have the same).
+template <int QT, bool X, bool TWO>
 __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K;
@@ -1034,7 +1037,7 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
     GgItems it(a, chunks, chunks);
     if (!it.next()) return;
     // superblocks of `it`'s rows
-    auto superblocks = [&]() __attribute__((always_inline)) { return it.e == a.E ? a.nsb_sh : a.nsb; };
+    auto superblocks = [&]() __attribute__((always_inline)) { return TWO && it.e == a.E ? a.nsb_sh : a.nsb; };
     // the item's matrix from the wave's first row; blocks past the end
     // repeat the last one and are not stored
     auto matrix = [&]() __attribute__((always_inline)) {
@@ -1043,12 +1046,13 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
     auto block_row = [&](int chunk, int blk) __attribute__((always_inline)) {
         return chunk * DN_ROWS + 32 * (DN_BLOCKS * w + blk);
     };
-    // piece 64 j + lane of a unit: its row and the piece's offset
+    // piece 64 j + lane of a unit: its row (its offset unless TWO) and the
+    // piece's offset
     uint32_t ro[UNIT_LD<QT>], po[UNIT_LD<QT>];
 #pragma unroll
     for (int j = 0; j < UNIT_LD<QT>; j++) {
         const uint32_t c = (uint32_t)min(64 * j + lane, 32 * ROW_CH<QT> - 1);
-        ro[j] = c / ROW_CH<QT>;
+        ro[j] = c / ROW_CH<QT> * (TWO ? 1u : (uint32_t)a.nsb * Raw<QT>::BYTES);
         po[j] = 16 * min(c % ROW_CH<QT>, (uint32_t)(QT == Q4 ? 8 : 13));
     }
     // unit u: block u / nb, superblock u % nb
@@ -1058,7 +1062,8 @@ __global__ __launch_bounds__(DN_WAVES * WAVE, 2) void k_down_gg(const GgArgs a)
         const uint8_t *p = m + (uint64_t)(uint32_t)min(block_row(chunk, blk), a.rows - 32) * rb;
 #pragma unroll
         for (int j = 0; j < UNIT_LD<QT>; j++)
-            lds_load16(p + (((ro[j] * rb + (uint32_t)b * Raw<QT>::BYTES) & ~15u) + po[j]), &sW[w][64 * j]);
+            lds_load16(p + ((((TWO ? ro[j] * rb : ro[j]) + (uint32_t)b * Raw<QT>::BYTES) & ~15u) + po[j]),
+                       &sW[w][64 * j]);
     };
     // 16 threads a token, each the units q + 16 k of its superblocks
     const int hn = tid >> 4, hq = tid & 15;
@@ -1265,9 +1270,11 @@ void launch_down(const GgArgs &a, int td, bool exact, int tiles, int cus, hipStr
 {
     constexpr int Q4 = BREAD_QTYPE_Q4_K, Q6 = BREAD_QTYPE_Q6_K;
     const dim3 grid = gg_grid(tiles, (a.rows + DN_ROWS - 1) / DN_ROWS, cus), block(DN_WAVES * WAVE);
-    if (!exact) hipLaunchKernelGGL((k_down_gg<Q6, false>), grid, block, 0, st, a);
-    else if (td == Q4) hipLaunchKernelGGL((k_down_gg<Q4, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((k_down_gg<Q6, true>), grid, block, 0, st, a);
+    const bool two = a.nsb != a.nsb_sh;
+    const auto kernel = !exact     ? (two ? k_down_gg<Q6, false, true> : k_down_gg<Q6, false, false>)
+                        : td == Q4 ? (two ? k_down_gg<Q4, true, true> : k_down_gg<Q4, true, false>)
+                                   : (two ? k_down_gg<Q6, true, true> : k_down_gg<Q6, true, false>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, a);
 }
 
 }  // namespace
